@@ -41,6 +41,7 @@ SOURCES = [
     "kernels/gemm.hip",
     "kernels/gemm_mfma.hip",
     "kernels/gemm_q.hip",
+    "kernels/gemm_skinny.hip",
     "kernels/gemma.hip",
     "kernels/chain.hip",
     "kernels/noalloc.hip",

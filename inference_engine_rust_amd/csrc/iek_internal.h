@@ -51,8 +51,25 @@ struct MvSegDesc {
 void launch_matvec(int dt, const MvSegDesc* segs, int nseg, const float* x, int K, int epi, hipStream_t st);
 void launch_gemm(int dt, const void* w, const float* a, int M, int K, int N, float* out, const float* resid,
                  hipStream_t st);
+// A prefill GEMM input of M rows and K columns (K % 32 == 0) is two fp16 planes (hi, lo) in the
+// order the matrix-core GEMMs read them: 16-row x 32-column tiles, K-major within a row tile, each
+// tile's 16 rows of 64 bytes back to back (plane_chunk), each 16-byte chunk of eight values in the
+// order 0, 2, 1, 3, 4, 6, 5, 7 (the order in which masking a dword's bytes 0 and 2, then 1 and 3,
+// yields the weights). Rows past M of the last row tile are never
+// written; they reach only output rows that are not stored. Against row-major planes, whose rows
+// of a power-of-two width all start on one memory channel: the few-row GEMM of 13 x 14336 x 4096
+// took 42 us, with the tiles 35.
+__host__ __device__ inline size_t plane_halves(int M, int K) { return (size_t)((M + 15) / 16 * 16) * K; }
+// 16-byte chunk index of row m, columns 8 k8 .. 8 k8 + 7 (kb = K / 32)
+__host__ __device__ inline size_t plane_chunk(int m, int k8, int kb) {
+  return ((size_t)(m >> 4) * kb + (k8 >> 2)) * 64 + 4 * (m & 15) + (k8 & 3);
+}
+// position of value i (0..7) within its chunk; its own inverse
+__host__ __device__ constexpr int plane_pos(int i) { return (i & 4) | ((i & 1) << 1) | ((i >> 1) & 1); }
+// where per-32 sum b of a row of kb goes: plane_pos order within whole groups of eight (a partial
+// last group keeps its order; the weights that read sums have K % 256 == 0)
+__host__ __device__ inline int sums_pos(int b, int kb) { return (b | 7) < kb ? (b & ~7) + plane_pos(b & 7) : b; }
 // Matrix-core GEMM on activations pre-split into fp16 pairs (kernels/gemm_mfma.hip).
-void launch_split_f16(const float* x, size_t n, __half* hi, __half* lo, hipStream_t st);
 bool gemm_mfma_ok(int dt, const void* w, int K, int N);
 // Matrix-core GEMM for K-quant / Q8_0 weights with block scales applied outside the fp16 operands
 // (kernels/gemm_q.hip); up to three weight matrices sharing the activation in one launch.
@@ -61,23 +78,40 @@ struct GemmQSeg {
   float* out;
   int n;
 };
+// Scratch of the few-row kernel's K split: SK_MAX_GROUPS counters, zero before the first call (the
+// kernel leaves them zero), and sk_part_floats() floats of partial sums (256 column groups and K
+// parts of 64 columns per 16 rows). Calls that share them are ordered by their stream. Without it
+// (null) K is not split over workgroups.
+constexpr int SK_MAX_GROUPS = 1024, SK_MAX_ROWS = 256;
+struct SkScratch {
+  int* cnt;
+  float* part;
+};
+inline size_t sk_part_floats(int M) {
+  return M > SK_MAX_ROWS ? 0 : (size_t)256 * 1024 * (M <= 32 ? (M + 15) / 16 : 4 * ((M + 63) / 64));
+}
 bool gemm_q_ok(int dt, const void* w, int K);
 int num_cus();  // compute units of the current device
-void launch_block_sums(const float* a, int M, int K, float* xs, hipStream_t st);
 // kpart: optional M x N f32 scratch; with it a one-segment K-quant GEMM whose tiles would fill at
 // most half the CUs splits K in two and adds the second half's partial sums in a second pass; with
 // defer_add that pass is left to the caller (true is returned while kpart holds the partial sums:
 // out + kpart is the result, e.g. through launch_rmsnorm_split's `part`).
 bool launch_gemm_q(int dt, const GemmQSeg* segs, int nseg, const __half* xh, const __half* xl, const float* xs, int M,
-                   int K, const float* resid, hipStream_t st, float* kpart = nullptr, bool defer_add = false);
+                   int K, const float* resid, hipStream_t st, float* kpart = nullptr, bool defer_add = false,
+                   const float* row_scale = nullptr, const SkScratch* sk = nullptr);
+// Whether launch_gemm_q takes M rows against N weight columns (all segments together) through the
+// few-row kernel (gemm_skinny.hip), which also applies row_scale and reads native Q6_K.
+bool gemm_skinny_ok(int dt, int M, int N);
+// Whether it splits the K of an N-column weight over workgroups (and so takes an SkScratch).
+bool gemm_skinny_splits(int K, int N);
 // Gate/up projection with SwiGLU in its epilogue (K-quant Q4_K or regrouped Q6_K weights of equal
 // shape, N % 32 == 0): writes act = silu(x W_gate^T) * (x W_up^T) as the down projection's input,
-// the fp16 (hi, lo) planes [M][N], optionally their per-32 sums (as launch_swiglu_split's `sums`)
+// the fp16 (hi, lo) planes, optionally their per-32 sums (as launch_swiglu_split's `sums`)
 // and the f32 act; the same bits as launch_gemm_q into gate and up followed by launch_swiglu_split.
 // Returns false, launching nothing, for other weight types or shapes.
 bool launch_gemm_q_glu(int dt, const void* w_gate, const void* w_up, int N, const __half* xh, const __half* xl,
                        const float* xs, int M, int K, __half* act_hi, __half* act_lo, float* act_sums, float* act_f32,
-                       int* ovf, hipStream_t st);
+                       int* ovf, hipStream_t st, const SkScratch* sk = nullptr);
 // out[i] += part[i] for i < n (n % 4 == 0, 16-byte aligned)
 void launch_add_f32(float* out, const float* part, size_t n, hipStream_t st);
 void launch_gemm_mfma(int dt, const void* w, const __half* xh, const __half* xl, int M, int K, int N, float* out,
@@ -88,8 +122,8 @@ void launch_embed(int dt, const void* table, size_t hidden, size_t rows, const u
                   float* out, hipStream_t st);
 void launch_rmsnorm(const float* in, const float* w, int rows, int dim, float eps, float* out, hipStream_t st);
 // Producers that also emit a prefill GEMM input: fp16 (hi, lo) planes of their [rows, dim] output
-// and its per-32 sums as an fp16 pair (two planes of rows * dim / 32 halves at `sums`), as
-// launch_split_f16 + launch_block_sums would (dim % 32 == 0, 16-byte aligned rows). A null `out`
+// (plane_chunk) and its per-32 sums as an fp16 pair (two row-major planes of rows * dim / 32 halves
+// at `sums`, in plane_pos order within each group of eight); dim % 32 == 0, 16-byte aligned rows. A null `out`
 // skips the f32 output. With `part`, in[i] + part[i] (one f32 add, as launch_add_f32) is
 // normalised and written back to `in`. A value or per-32 sum beyond the pair's range (F16_PAIR_MAX)
 // sets *ovf (when given).
@@ -107,8 +141,9 @@ void launch_range_flag(const float* a, size_t n, int* ovf, hipStream_t st);
 // the fp16 (hi, lo) planes of s * a and the per-32 sums of s * a (fp16 pair planes), and
 // inv[m] = 1 / s. Then launch_row_scale multiplies each output row by inv[m]; power-of-two factors
 // make both steps exact.
-void launch_split_scaled(const float* a, int rows, int K, __half* hi, __half* lo, float* sums, float* inv,
-                         hipStream_t st);
+// With `cnt`, `ncnt` ints there are cleared.
+void launch_split_scaled(const float* a, int rows, int K, __half* hi, __half* lo, float* sums, float* inv, int* cnt,
+                         int ncnt, hipStream_t st);
 void launch_row_scale(float* out, int rows, int N, const float* inv, hipStream_t st);
 // Prefill attention on f32 inputs (the path taken when an input is beyond the fp16 pair's range):
 // q [M][n_heads*hd], k and v [M][n_kv*hd] (RoPE applied), causal over the M prompt rows with the

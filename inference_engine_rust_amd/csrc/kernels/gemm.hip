@@ -77,19 +77,27 @@ void launch_gemm(int dt, const void* w, const float* a, int M, int K, int N, flo
   }
   // stream-ordered scratch: the fp16 pair, the per-32 sums, the row factors, a split-K partial and
   // (Q6_K) the regrouped weights
-  const size_t n = (size_t)M * K;
-  const bool q6r = kq && dt == DT_Q6K && K % QK_K == 0;
+  const size_t n = plane_halves(M, K), nb = (size_t)M * (K / 32);
+  const bool skinny = kq && gemm_skinny_ok(dt, M, N);
+  const bool q6r = kq && !skinny && dt == DT_Q6K && K % QK_K == 0;
   const size_t wr = q6r ? (size_t)N * q6r_row_bytes((size_t)K / QK_K) : 0;
-  const size_t xbytes = (n * 2 * sizeof(__half) + (n / 32 + 64) * sizeof(float) + 255) / 256 * 256;
+  const size_t xbytes = (n * 2 * sizeof(__half) + (nb + 64) * sizeof(float) + 255) / 256 * 256;
   const size_t ibytes = ((size_t)M * sizeof(float) + 255) / 256 * 256;
-  const size_t pbytes = kq ? ((size_t)M * N * sizeof(float) + 255) / 256 * 256 : 0;  // split-K partial
+  // split-K partials (the few-row kernel's behind its arrival counters)
+  const bool sks = skinny && gemm_skinny_splits(K, N);
+  const size_t pbytes = sks      ? SK_MAX_GROUPS * sizeof(int) + sk_part_floats(M) * sizeof(float)
+                        : skinny ? 0
+                        : kq     ? ((size_t)M * N * sizeof(float) + 255) / 256 * 256
+                                 : 0;
   void* buf = nullptr;
   check_hip(hipMallocAsync(&buf, xbytes + ibytes + pbytes + wr, st), "hipMallocAsync");
   char* base = static_cast<char*>(buf);
   __half* xh = reinterpret_cast<__half*>(base);
   float* xs = reinterpret_cast<float*>(xh + 2 * n);
   float* inv = reinterpret_cast<float*>(base + xbytes);
-  launch_split_scaled(a, M, K, xh, xh + n, xs, inv, st);
+  SkScratch sk{reinterpret_cast<int*>(base + xbytes + ibytes), nullptr};
+  sk.part = reinterpret_cast<float*>(sk.cnt + SK_MAX_GROUPS);
+  launch_split_scaled(a, M, K, xh, xh + n, xs, inv, sks ? sk.cnt : nullptr, SK_MAX_GROUPS, st);
   if (kq) {
     const void* wq = w;
     int wdt = dt;
@@ -100,11 +108,12 @@ void launch_gemm(int dt, const void* w, const float* a, int M, int K, int N, flo
       wdt = DT_Q6K_R;
     }
     GemmQSeg seg{wq, out, N};
-    launch_gemm_q(wdt, &seg, 1, xh, xh + n, xs, M, K, nullptr, st, reinterpret_cast<float*>(base + xbytes + ibytes));
+    launch_gemm_q(wdt, &seg, 1, xh, xh + n, xs, M, K, nullptr, st, reinterpret_cast<float*>(base + xbytes + ibytes),
+                  false, skinny ? inv : nullptr, sks ? &sk : nullptr);
   } else {
     launch_gemm_mfma(dt, w, xh, xh + n, M, K, N, out, nullptr, st);
   }
-  launch_row_scale(out, M, N, inv, st);
+  if (!skinny) launch_row_scale(out, M, N, inv, st);
   check_hip(hipFreeAsync(buf, st), "hipFreeAsync");
 }
 

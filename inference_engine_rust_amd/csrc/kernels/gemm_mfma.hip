@@ -43,27 +43,9 @@ IEK_DEV void split8(const float (&v)[8], uint4& hi, uint4& lo) {
     h[i] = (_Float16)v[i];
     l[i] = (_Float16)(v[i] - (float)h[i]);
   }
-  hi = make_uint4(pack2(h[0], h[1]), pack2(h[2], h[3]), pack2(h[4], h[5]), pack2(h[6], h[7]));
-  lo = make_uint4(pack2(l[0], l[1]), pack2(l[2], l[3]), pack2(l[4], l[5]), pack2(l[6], l[7]));
-}
-
-__global__ __launch_bounds__(256) void split_f16_kernel(const float* __restrict__ x, size_t n8, uint4* __restrict__ hi,
-                                                        uint4* __restrict__ lo) {
-  for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n8; i += (size_t)gridDim.x * 256) {
-    const float4 a = reinterpret_cast<const float4*>(x)[2 * i], b = reinterpret_cast<const float4*>(x)[2 * i + 1];
-    const float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
-    uint4 h, l;
-    split8(v, h, l);
-    hi[i] = h;
-    lo[i] = l;
-  }
-}
-
-void launch_split_f16(const float* x, size_t n, __half* hi, __half* lo, hipStream_t st) {
-  if (n % 8 != 0) fail(ST_OP, "split_f16: length must be a multiple of 8");
-  const size_t n8 = n / 8;
-  const int blocks = (int)std::min<size_t>((n8 + 255) / 256, 4096);
-  hipLaunchKernelGGL(split_f16_kernel, dim3(std::max(blocks, 1)), dim3(256), 0, st, x, n8, (uint4*)hi, (uint4*)lo);
+  // the order of the activation planes (plane_pos)
+  hi = make_uint4(pack2(h[0], h[2]), pack2(h[1], h[3]), pack2(h[4], h[6]), pack2(h[5], h[7]));
+  lo = make_uint4(pack2(l[0], l[2]), pack2(l[1], l[3]), pack2(l[4], l[6]), pack2(l[5], l[7]));
 }
 
 // ---- exact dequantisation of 8 consecutive flat elements f0 .. f0+7 (f0 % 8 == 0) ----------
@@ -168,7 +150,7 @@ IEK_DEV void fetch_a(const __half* xh, const __half* xl, int m0, int M, int K, i
 #pragma unroll
   for (int u = 0; u < AU; ++u) {
     const int idx = tid + 256 * u, row = idx >> 2, c8 = idx & 3;
-    const size_t off = (size_t)min(m0 + row, M - 1) * K + k0 + 8 * c8;
+    const size_t off = 8 * plane_chunk(min(m0 + row, M - 1), k0 / 8 + c8, K / 32);
     arh[u] = *reinterpret_cast<const u4_t*>(xh + off);
     arl[u] = *reinterpret_cast<const u4_t*>(xl + off);
   }

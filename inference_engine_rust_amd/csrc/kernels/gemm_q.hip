@@ -19,42 +19,12 @@
 // share the activation (Q/K/V) run as one launch; M tiles of one N tile share an XCD's L2.
 #include <cstdlib>
 
-#include "common.cuh"
+#include "kq_core.cuh"
 #include "../iek_internal.h"
 
 namespace iek {
 
-struct GemmQArgs {
-  const uint8_t* w[3];
-  float* out[3];
-  int n[3];
-  int tile_start[4];  // first N tile of each segment; tile_start[nseg] = total N tiles
-  int nseg;
-  int M, K;
-  size_t row_bytes;
-  const __half* xh;
-  const __half* xl;
-  const float* xs;
-  const float* resid;  // segment 0 only
-  int xcd_remap;
-  // split-K (wave-tiled kernel, one segment): the second half of the superblocks writes its
-  // partial sums to kpart [M, N], which a follow-up pass adds to out
-  int ksplit;
-  float* kpart;
-  // gate/up + SwiGLU (wave-tiled kernel instantiated with GLU, segments 0 = gate and 1 = up of
-  // equal N): each wave computes 32 gate and the same 32 up columns; the epilogue writes
-  // act = silu(gate) * up as the down projection's input: fp16 (hi, lo) planes [M][N], their
-  // per-32 sums (glu_sums, optional) and the f32 act (glu_out, optional)
-  _Float16 *glu_h, *glu_l, *glu_sums;
-  float* glu_out;
-  int* ovf;  // GLU: set when an act value or per-32 sum is beyond the fp16 pair's range
-};
-
 namespace {
-
-typedef _Float16 qh8_t __attribute__((ext_vector_type(8)));
-typedef float qf4_t __attribute__((ext_vector_type(4)));
-typedef uint32_t qu4_t __attribute__((ext_vector_type(4)));
 
 constexpr int QBK = 32, QROW = 40;  // K per stage, LDS row (halves, padded)
 
@@ -101,8 +71,8 @@ struct QDeq<DT_Q6K> {
       h[i] = (_Float16)wq;
       l[i] = (_Float16)(wq - (int)h[i]);
     }
-    hi = make_uint4(hpack(h[0], h[1]), hpack(h[2], h[3]), hpack(h[4], h[5]), hpack(h[6], h[7]));
-    lo = make_uint4(hpack(l[0], l[1]), hpack(l[2], l[3]), hpack(l[4], l[5]), hpack(l[6], l[7]));
+    hi = make_uint4(hpack(h[0], h[2]), hpack(h[1], h[3]), hpack(h[4], h[6]), hpack(h[5], h[7]));  // plane_pos order
+    lo = make_uint4(hpack(l[0], l[2]), hpack(l[1], l[3]), hpack(l[4], l[6]), hpack(l[5], l[7]));
   }
 };
 
@@ -123,29 +93,10 @@ struct QDeq<DT_Q8_0> {
     _Float16 h[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) h[i] = (_Float16)(int)(int8_t)((q[i >> 1] >> (8 * (i & 1))) & 0xFFu);
-    hi = make_uint4(hpack(h[0], h[1]), hpack(h[2], h[3]), hpack(h[4], h[5]), hpack(h[6], h[7]));
+    hi = make_uint4(hpack(h[0], h[2]), hpack(h[1], h[3]), hpack(h[4], h[6]), hpack(h[5], h[7]));  // plane_pos order
     lo = make_uint4(0, 0, 0, 0);
   }
 };
-
-// Per-32 row sums of the activation (Q4_K's min term), summed in f32 and stored as an fp16 pair
-// over two planes of nb halves: hi[m * (K/32) + b] + lo[...] = sum of a[m, 32b .. 32b+31].
-__global__ __launch_bounds__(256) void block_sums_kernel(const float* __restrict__ a, size_t nb,
-                                                         _Float16* __restrict__ hi, _Float16* __restrict__ lo) {
-#pragma clang fp contract(off)
-  const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-  if (i >= nb) return;
-  const float4* p = reinterpret_cast<const float4*>(a + 32 * i);
-  float s = 0.f;
-#pragma unroll
-  for (int t = 0; t < 8; ++t) {
-    const float4 v = p[t];
-    s += (v.x + v.y) + (v.z + v.w);
-  }
-  const _Float16 h = (_Float16)s;
-  hi[i] = h;
-  lo[i] = (_Float16)(s - (float)h);
-}
 
 template <int DT, int BM, int BN>
 __global__ __launch_bounds__(256) void gemm_q_kernel(GemmQArgs g) {
@@ -208,7 +159,7 @@ __global__ __launch_bounds__(256) void gemm_q_kernel(GemmQArgs g) {
 #pragma unroll
     for (int u = 0; u < AU; ++u) {
       const int idx = tid + 256 * u, row = idx >> 2, c8 = idx & 3;
-      const size_t off = (size_t)min(m0 + row, M - 1) * K + k0 + 8 * c8;
+      const size_t off = 8 * plane_chunk(min(m0 + row, M - 1), k0 / 8 + c8, K / 32);
       sl.arh[u] = *reinterpret_cast<const qu4_t*>(g.xh + off);
       sl.arl[u] = *reinterpret_cast<const qu4_t*>(g.xl + off);
     }
@@ -333,48 +284,6 @@ __global__ __launch_bounds__(256) void gemm_q_kernel(GemmQArgs g) {
 // lane's own weight column, so the superblock factors d and dmin apply per lane. The min term
 // -dmin * sum_b m_b * sum(a over sub-block b) runs on the matrix cores once per superblock: the
 // per-32 activation sums (fp16 pair) against the eight 6-bit mins.
-typedef _Float16 qh2_t __attribute__((ext_vector_type(2)));
-
-IEK_DEV uint32_t pk_fma16(uint32_t a, uint32_t b, uint32_t c) {
-  return __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(__builtin_bit_cast(qh2_t, a), __builtin_bit_cast(qh2_t, b),
-                                                                __builtin_bit_cast(qh2_t, c)));
-}
-// (1024 + byte) as fp16 in each half: bytes of x picked by the selector's bytes 0 and 2.
-IEK_DEV uint32_t mag16(uint32_t x, uint32_t sel) { return __builtin_amdgcn_perm(0x64646464u, x, sel); }
-constexpr uint32_t SEL01 = 0x04010400u, SEL23 = 0x04030402u;
-constexpr uint32_t H2_M1024 = 0xE400E400u;  // (-1024, -1024)
-constexpr uint32_t H2_ONE = 0x3C003C00u;    // (1, 1)
-
-// {sc, sc} and {-1024 sc, -1024 sc} for the 6-bit scale in byte `i` of `scs`.
-IEK_DEV void q4k_scale2(uint32_t scs, uint32_t i, uint32_t& s2, uint32_t& c2) {
-  s2 = pk_fma16(mag16(scs, 0x04000400u | i | (i << 16)), H2_ONE, H2_M1024);
-  c2 = pk_fma16(s2, H2_M1024, 0u);
-}
-
-// B operand of sub-block 2P + H (H = 0: low nibbles, 1: high nibbles) for one 16-column tile.
-template <int P, int H>
-IEK_DEV qu4_t q4k_b(const uint4& hdr, uint2 q) {
-  const uint32_t scs = P < 2 ? (hdr.y & 0x3F3F3F3Fu) : ((hdr.w & 0x0F0F0F0Fu) | ((hdr.y >> 2) & 0x30303030u));
-  uint32_t sc, c;
-  q4k_scale2(scs, 2 * (P & 1) + H, sc, c);
-  const uint32_t x = (q.x >> (4 * H)) & 0x0F0F0F0Fu, y = (q.y >> (4 * H)) & 0x0F0F0F0Fu;
-  return qu4_t{pk_fma16(mag16(x, SEL01), sc, c), pk_fma16(mag16(x, SEL23), sc, c), pk_fma16(mag16(y, SEL01), sc, c),
-               pk_fma16(mag16(y, SEL23), sc, c)};
-}
-
-// The eight 6-bit mins of a superblock as fp16 (k groups 0 and 1; zero for groups 2 and 3).
-IEK_DEV qu4_t q4k_mins(const uint4& hdr, bool live) {
-  const uint32_t m03 = hdr.z & 0x3F3F3F3Fu;
-  const uint32_t m47 = ((hdr.w >> 4) & 0x0F0F0F0Fu) | ((hdr.z >> 2) & 0x30303030u);
-  qu4_t r{pk_fma16(mag16(m03, SEL01), H2_ONE, H2_M1024), pk_fma16(mag16(m03, SEL23), H2_ONE, H2_M1024),
-          pk_fma16(mag16(m47, SEL01), H2_ONE, H2_M1024), pk_fma16(mag16(m47, SEL23), H2_ONE, H2_M1024)};
-  return live ? r : qu4_t{0u, 0u, 0u, 0u};
-}
-
-IEK_DEV qf4_t mfma16(qu4_t a, qu4_t b, qf4_t c) {
-  return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(qh8_t, a), __builtin_bit_cast(qh8_t, b), c, 0, 0, 0);
-}
-
 // Buffer resource over `bytes` bytes at `p` (raw, unswizzled; word 3 as gfx9 data loads expect).
 IEK_DEV __amdgpu_buffer_rsrc_t buf_rsrc(const void* p, uint32_t bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), (short)0, (int)bytes, 0x00020000);
@@ -482,7 +391,7 @@ struct Q6RB {
       const uint2 l = H ? q.l1[j] : q.l0[j], hb = q.h[j];
       const uint32_t qx = ((l.x >> (4 * (P & 1))) & 0x0F0F0F0Fu) | (((hb.x >> (2 * qd)) << 4) & 0x30303030u);
       const uint32_t qy = ((l.y >> (4 * (P & 1))) & 0x0F0F0F0Fu) | (((hb.y >> (2 * qd)) << 4) & 0x30303030u);
-      const uint32_t v[4] = {mag16(qx, SEL01), mag16(qx, SEL23), mag16(qy, SEL01), mag16(qy, SEL23)};
+      const uint32_t v[4] = {mag16(qx, SEL02), mag16(qx, SEL13), mag16(qy, SEL02), mag16(qy, SEL13)};
       uint32_t hi[4], lo[4];
 #pragma unroll
       for (int t = 0; t < 4; ++t) {
@@ -517,78 +426,6 @@ IEK_DEV void kq_deq(int p, int h, const typename T::Hdr& hd, const typename T::R
     case 6: T::template deq<3, 0>(hd, q, bh, bl); break;
     default: T::template deq<3, 1>(hd, q, bh, bl); break;
   }
-}
-
-// SwiGLU epilogue of a gate/up tile (GLU): column groups 0-1 of a wave are gate columns and 2-3
-// the same up columns, so each lane holds matching gate / up sums. act = silu(g) * u with the
-// arithmetic of swiglu_split_kernel (src/ops/swiglu.rs:24-36: two-branch stable sigmoid,
-// (g * s) * u), then its fp16 (hi, lo) pair and, per 32 columns, the sum in emit_split8's order
-// (pairs, pairs of pairs, then the eight quarter sums one after the other from zero), so the down
-// projection's input has the bits the separate pass would write.
-// (Staging the fp16 pair through LDS for 16-byte stores measured no faster.)
-template <int TM, typename AccT>
-IEK_DEV void glu_epilogue(const GemmQArgs& g, const AccT& acc, const float (&Dc)[4], bool rescaled, int m0, int wcol,
-                          int lane) {
-#pragma clang fp contract(off)
-  const int lr = lane & 15, lg = lane >> 4;
-  const int M = g.M, N = g.n[0];
-  const size_t nb = (size_t)N / 32;
-  bool big = false;
-#pragma unroll
-  for (int i = 0; i < TM; ++i)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int m = m0 + 16 * i + 4 * lg + r;
-      float vv[2];
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        const int n = wcol + 16 * j + lr;
-        const float x = rescaled ? acc[i][j][r] * Dc[j] : acc[i][j][r];
-        const float u = rescaled ? acc[i][j + 2][r] * Dc[j + 2] : acc[i][j + 2][r];
-        float sg;
-        if (x >= 0.0f) {
-          const float z = expf(-x);
-          sg = 1.0f / (1.0f + z);
-        } else {
-          const float z = expf(x);
-          sg = z / (1.0f + z);
-        }
-        const float v = x * sg * u;
-        if (m < M && n < N) {
-          const size_t o = (size_t)m * N + n;
-          const _Float16 h = (_Float16)v;
-          g.glu_h[o] = h;
-          g.glu_l[o] = (_Float16)(v - (float)h);
-          if (g.glu_out) g.glu_out[o] = v;
-          big |= fabsf(v) > F16_PAIR_MAX;
-        }
-        vv[j] = v;
-      }
-      if (g.glu_sums) {
-        // (v0 + v1) + (v2 + v3) over each aligned group of four columns, at the group's first lane
-        float qs[2];
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-          const float s1 = vv[j] + __shfl_xor(vv[j], 1, 64);
-          qs[j] = s1 + __shfl_xor(s1, 2, 64);
-        }
-        // the wave's 32 columns are one block; its eight quarter sums sit at lanes 0, 4, 8, 12 of
-        // the lane's row of 16 (same m) for j = 0, then j = 1
-        float sum = 0.f;
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-          for (int t = 0; t < 4; ++t) sum += __shfl(qs[j], (lane & ~15) + 4 * t, 64);
-        if (lr == 0 && m < M && wcol < N) {
-          const size_t o = (size_t)m * nb + wcol / 32;
-          const _Float16 h = (_Float16)sum;
-          g.glu_sums[o] = h;
-          g.glu_sums[(size_t)M * nb + o] = (_Float16)(sum - (float)h);
-          big |= fabsf(sum) > F16_PAIR_MAX;
-        }
-      }
-    }
-  if (big && g.ovf) *g.ovf = 1;
 }
 
 // TM: 16-row MFMA tiles per wave along M (a wave owns 16 TM x 64); WGM x WGN waves.
@@ -644,17 +481,25 @@ __global__ __launch_bounds__(64 * WGM * WGN, OCC) void gemm_kq_kernel(GemmQArgs 
   // stage's advance in the scalar offset.
   const __amdgpu_buffer_rsrc_t rw = buf_rsrc(w, (uint32_t)(g.row_bytes * (size_t)N));
   const __amdgpu_buffer_rsrc_t rw2 = GLU ? buf_rsrc(g.w[1], (uint32_t)(g.row_bytes * (size_t)N)) : rw;
-  const __amdgpu_buffer_rsrc_t rxh = buf_rsrc(g.xh, (uint32_t)((size_t)M * K * 2));
-  const __amdgpu_buffer_rsrc_t rxl = buf_rsrc(g.xl, (uint32_t)((size_t)M * K * 2));
+  const __amdgpu_buffer_rsrc_t rxh = buf_rsrc(g.xh, (uint32_t)(plane_halves(M, K) * 2));
+  const __amdgpu_buffer_rsrc_t rxl = buf_rsrc(g.xl, (uint32_t)(plane_halves(M, K) * 2));
   const __amdgpu_buffer_rsrc_t rxs = buf_rsrc(g.xs, T::MINS ? (uint32_t)((size_t)M * kb * 4) : 0u);
   uint32_t vb[4];  // weight row of the lane's column in each 16-column tile
 #pragma unroll
   for (int j = 0; j < 4; ++j)
     vb[j] = (uint32_t)((size_t)min(wcol + 16 * (GLU ? (j & 1) : j) + lr, N - 1) * g.row_bytes);
-  uint32_t va[AR];  // activation rows staged by this thread (both planes)
+  // activation chunks staged by this thread (both planes): chunk i = tid + NT u of the stage's BM
+  // rows x 64 columns is row tile i >> 7, column tile (i >> 6) & 1, chunk i & 63 within the tile
+  uint32_t va[AR];
+  int as_row[AR], as_c[AR];
 #pragma unroll
-  for (int u = 0; u < AR; ++u)
-    va[u] = (uint32_t)(min(m0 + (tid >> 3) + (NT / 8) * u, M - 1) * K + 8 * (tid & 7)) * 2u;
+  for (int u = 0; u < AR; ++u) {
+    const int i = tid + NT * u;
+    as_row[u] = 16 * (i >> 7) + ((i & 63) >> 2);
+    as_c[u] = 4 * ((i >> 6) & 1) + (i & 3);
+    const int rt = min((m0 >> 4) + (i >> 7), (M - 1) >> 4);
+    va[u] = (((uint32_t)rt * kb + ((i >> 6) & 1)) * 64 + (i & 63)) * 16u;
+  }
   uint32_t vx[TM];  // per-32 sums: k group 0 reads the hi plane, 1 the lo plane
 #pragma unroll
   for (int i = 0; i < TM; ++i)
@@ -671,17 +516,16 @@ __global__ __launch_bounds__(64 * WGM * WGN, OCC) void gemm_kq_kernel(GemmQArgs 
   auto fetch_a = [&](int kt, ASlot& sl) {
 #pragma unroll
     for (int u = 0; u < AR; ++u) {
-      sl.a[u] = ld_b128(rxh, va[u], 128u * kt);
-      sl.a[AR + u] = ld_b128(rxl, va[u], 128u * kt);
+      sl.a[u] = ld_b128(rxh, va[u], 2048u * kt);
+      sl.a[AR + u] = ld_b128(rxl, va[u], 2048u * kt);
     }
   };
   auto store_a = [&](int buf, const ASlot& sl) {
-    const int c = tid & 7;
 #pragma unroll
     for (int u = 0; u < AR; ++u) {
-      const int row = (tid >> 3) + (NT / 8) * u;
-      As[buf][row * 8 + (c ^ (row & 7))] = sl.a[u];
-      As[buf][PL + row * 8 + (c ^ (row & 7))] = sl.a[AR + u];
+      const int ch = as_row[u] * 8 + (as_c[u] ^ (as_row[u] & 7));
+      As[buf][ch] = sl.a[u];
+      As[buf][PL + ch] = sl.a[AR + u];
     }
   };
   auto fetch_xs = [&](int sb) {
@@ -900,13 +744,6 @@ bool gemm_q_ok(int dt, const void* w, int K) {
   }
 }
 
-void launch_block_sums(const float* a, int M, int K, float* xs, hipStream_t st) {
-  if (K % 32 != 0) fail(ST_OP, "block_sums: K must be a multiple of 32");
-  const size_t nb = (size_t)M * (K / 32);
-  _Float16* h = reinterpret_cast<_Float16*>(xs);
-  hipLaunchKernelGGL(block_sums_kernel, dim3((unsigned)((nb + 255) / 256)), dim3(256), 0, st, a, nb, h, h + nb);
-}
-
 template <int DT, int BM, int BN>
 static void gemm_q_launch(GemmQArgs g, hipStream_t st) {
   int t = 0;
@@ -979,7 +816,7 @@ static void gemm_q_dt(GemmQArgs g, hipStream_t st) {
 
 bool launch_gemm_q_glu(int dt, const void* w_gate, const void* w_up, int N, const __half* xh, const __half* xl,
                        const float* xs, int M, int K, __half* act_hi, __half* act_lo, float* act_sums, float* act_f32,
-                       int* ovf, hipStream_t st) {
+                       int* ovf, hipStream_t st, const SkScratch* sk) {
   if (dt != DT_Q4K && dt != DT_Q6K_R) return false;
   if (M < 1 || N < 32 || N % 32 != 0 || !gemm_q_ok(dt, w_gate, K) || !gemm_q_ok(dt, w_up, K)) return false;
   if (dt == DT_Q4K && !xs) fail(ST_OP, "gemm_q: Q4_K needs the per-32 activation sums");
@@ -1000,7 +837,11 @@ bool launch_gemm_q_glu(int dt, const void* w_gate, const void* w_up, int N, cons
   g.glu_sums = reinterpret_cast<_Float16*>(act_sums);
   g.glu_out = act_f32;
   g.ovf = ovf;
-  if (dt == DT_Q4K) gemm_kq<Q4KB, true>(g, st, false);
+  if (gemm_skinny_ok(dt, M, 2 * N)) {
+    g.kpart = sk ? sk->part : nullptr;
+    g.sk_cnt = sk ? sk->cnt : nullptr;
+    launch_gemm_skinny(dt, g, true, st);
+  } else if (dt == DT_Q4K) gemm_kq<Q4KB, true>(g, st, false);
   else gemm_kq<Q6RB, true>(g, st, false);
   return true;
 }
@@ -1014,7 +855,7 @@ void launch_add_f32(float* out, const float* part, size_t n, hipStream_t st) {
 }
 
 bool launch_gemm_q(int dt, const GemmQSeg* segs, int nseg, const __half* xh, const __half* xl, const float* xs, int M,
-                   int K, const float* resid, hipStream_t st, float* kpart, bool defer_add) {
+                   int K, const float* resid, hipStream_t st, float* kpart, bool defer_add, const float* row_scale, const SkScratch* sk) {
   if (nseg < 1 || nseg > 3 || M < 1) fail(ST_OP, "gemm_q: 1..3 segments and M >= 1");
   GemmQArgs g{};
   g.nseg = nseg;
@@ -1040,6 +881,15 @@ bool launch_gemm_q(int dt, const GemmQSeg* segs, int nseg, const __half* xh, con
     default: g.row_bytes = (size_t)(K / 32) * Q8_0_BYTES; break;
   }
   if (dt == DT_Q4K && !xs) fail(ST_OP, "gemm_q: Q4_K needs the per-32 activation sums");
+  int ncols = 0;
+  for (int i = 0; i < nseg; ++i) ncols += segs[i].n;
+  if (gemm_skinny_ok(dt, M, ncols)) {
+    g.row_scale = row_scale;
+    g.kpart = sk ? sk->part : nullptr;
+    g.sk_cnt = sk ? sk->cnt : nullptr;
+    launch_gemm_skinny(dt, g, false, st);
+    return false;
+  }
   switch (dt) {
     case DT_Q4K: return gemm_kq<Q4KB>(g, st, defer_add);
     case DT_Q6K: gemm_q_dt<DT_Q6K>(g, st); return false;

@@ -83,15 +83,16 @@ void launch_rmsnorm(const float* in, const float* w, int rows, int dim, float ep
 }
 
 // ---- GEMM inputs: fp16 pair planes and per-32 sums emitted by the producing kernel -----------
-// Eight consecutive values v = a[8i .. 8i+7] of a [rows, K] input (K % 32 == 0): hi = fp16(v),
+// Eight consecutive values v = a[m][8 k8 .. 8 k8 + 7] of a [rows, 32 kb] input: hi = fp16(v),
 // lo = fp16(v - hi), and the per-32 sum of the block they belong to, summed in the order the
 // stand-alone per-32 sum pass uses (eight float4 partials (x + y) + (z + w), left to right) and
 // stored as an fp16 pair. The four consecutive lanes of one block exchange their partials by
 // shuffles, so every lane of the wave calls this (`live` masks the stores).
 // A value or per-32 sum beyond fp16's range (|x| > 65504: its pair would not hold it) sets *ovf;
 // the prefill then runs again on f32 activations (Session::prefill).
-IEK_DEV void emit_split8(const float (&v)[8], size_t i, bool live, uint4* __restrict__ hi, uint4* __restrict__ lo,
-                         _Float16* __restrict__ sh, _Float16* __restrict__ sl, int* __restrict__ ovf) {
+IEK_DEV void emit_split8(const float (&v)[8], int m, int k8, int kb, bool live, uint4* __restrict__ hi,
+                         uint4* __restrict__ lo, _Float16* __restrict__ sh, _Float16* __restrict__ sl,
+                         int* __restrict__ ovf) {
 #pragma clang fp contract(off)
   _Float16 h[8], l[8];
   bool big = false;
@@ -105,8 +106,9 @@ IEK_DEV void emit_split8(const float (&v)[8], size_t i, bool live, uint4* __rest
     return (uint32_t)__builtin_bit_cast(uint16_t, a) | ((uint32_t)__builtin_bit_cast(uint16_t, b) << 16);
   };
   if (live) {
-    hi[i] = make_uint4(pk(h[0], h[1]), pk(h[2], h[3]), pk(h[4], h[5]), pk(h[6], h[7]));
-    lo[i] = make_uint4(pk(l[0], l[1]), pk(l[2], l[3]), pk(l[4], l[5]), pk(l[6], l[7]));
+    const size_t i = plane_chunk(m, k8, kb);
+    hi[i] = make_uint4(pk(h[0], h[2]), pk(h[1], h[3]), pk(h[4], h[6]), pk(h[5], h[7]));
+    lo[i] = make_uint4(pk(l[0], l[2]), pk(l[1], l[3]), pk(l[4], l[6]), pk(l[5], l[7]));
   }
   const float pa = (v[0] + v[1]) + (v[2] + v[3]), pb = (v[4] + v[5]) + (v[6] + v[7]);
   const int lane = threadIdx.x & 63, base = lane & ~3;
@@ -121,8 +123,9 @@ IEK_DEV void emit_split8(const float (&v)[8], size_t i, bool live, uint4* __rest
 #pragma unroll
     for (int t = 0; t < 8; ++t) sum += p[t];
     const _Float16 s16 = (_Float16)sum;
-    sh[i / 4] = s16;
-    sl[i / 4] = (_Float16)(sum - (float)s16);
+    const size_t o = (size_t)m * kb + sums_pos(k8 >> 2, kb);
+    sh[o] = s16;
+    sl[o] = (_Float16)(sum - (float)s16);
     big |= fabsf(sum) > F16_PAIR_MAX;
   }
   if (live && big && ovf) *ovf = 1;
@@ -194,7 +197,7 @@ __global__ __launch_bounds__(256) void rmsnorm_split_kernel(float* in, const flo
       reinterpret_cast<float4*>(y)[2 * c + 1] = make_float4(v[4], v[5], v[6], v[7]);
     }
     // emit_split8 exchanges across the group of four lanes: every lane joins
-    emit_split8(v, (size_t)blockIdx.x * n8 + c, live, hi, lo, sh, sl, ovf);
+    emit_split8(v, blockIdx.x, c, dim / 32, live, hi, lo, sh, sl, ovf);
   }
 }
 
@@ -219,7 +222,7 @@ void launch_rmsnorm_split(float* in, const float* w, int rows, int dim, float ep
 }
 
 // fp16 pair planes and per-32 sums of an existing [rows, K] input in one pass.
-__global__ __launch_bounds__(256) void split_sums_kernel(const float* __restrict__ a, size_t n8, uint4* hi, uint4* lo,
+__global__ __launch_bounds__(256) void split_sums_kernel(const float* __restrict__ a, size_t n8, uint32_t k8n, uint4* hi, uint4* lo,
                                                          _Float16* sh, _Float16* sl, int* ovf) {
   for (size_t i0 = (size_t)blockIdx.x * 256; i0 < n8; i0 += (size_t)gridDim.x * 256) {
     const size_t i = i0 + threadIdx.x;
@@ -227,7 +230,7 @@ __global__ __launch_bounds__(256) void split_sums_kernel(const float* __restrict
     const size_t c = live ? i : 0;
     const float4 xa = reinterpret_cast<const float4*>(a)[2 * c], xb = reinterpret_cast<const float4*>(a)[2 * c + 1];
     const float v[8] = {xa.x, xa.y, xa.z, xa.w, xb.x, xb.y, xb.z, xb.w};
-    emit_split8(v, c, live, hi, lo, sh, sl, ovf);
+    emit_split8(v, (int)(c / k8n), (int)(c % k8n), k8n / 4, live, hi, lo, sh, sl, ovf);
   }
 }
 
@@ -238,7 +241,8 @@ void launch_split_sums(const float* a, int rows, int K, __half* hi, __half* lo, 
   const size_t n8 = (size_t)rows * (K / 8), nb = n8 / 4;
   _Float16* s = reinterpret_cast<_Float16*>(sums);
   const int blocks = (int)std::min<size_t>((n8 + 255) / 256, 4096);
-  hipLaunchKernelGGL(split_sums_kernel, dim3(blocks), dim3(256), 0, st, a, n8, (uint4*)hi, (uint4*)lo, s, s + nb, ovf);
+  hipLaunchKernelGGL(split_sums_kernel, dim3(blocks), dim3(256), 0, st, a, n8, (uint32_t)(K / 8), (uint4*)hi, (uint4*)lo, s,
+                     s + nb, ovf);
 }
 
 // *ovf = 1 when some |a[i]| exceeds the fp16 pair's range (NaN does not count: it stays NaN on
@@ -257,36 +261,48 @@ void launch_range_flag(const float* a, size_t n, int* ovf, hipStream_t st) {
 }
 
 // Per-row scaled GEMM input (op level): one workgroup per row. Pass 1 finds the row's largest
-// |value| and |per-32 sum| (sums in the order of block_sums_kernel: (x + y) + (z + w) per float4,
+// |value| and |per-32 sum| (sums in the order of emit_split8: (x + y) + (z + w) per float4,
 // left to right); the factor s = 2^e (e <= 0) brings that maximum below 2^15 when it is not
 // already; pass 2 writes the fp16 (hi, lo) planes of s * a and s * sum (exact: a power of two).
-__global__ __launch_bounds__(256) void split_scaled_kernel(const float* __restrict__ a, int K, _Float16* __restrict__ hi,
-                                                           _Float16* __restrict__ lo, _Float16* __restrict__ sh,
-                                                           _Float16* __restrict__ sl, size_t nb_total,
-                                                           float* __restrict__ inv) {
+// Each thread takes chunks of eight of the row, as emit_split8 does; the first CPT stay in registers
+// between the two passes (wider rows are read again).
+template <int CPT>
+__global__ __launch_bounds__(256) void split_scaled_kernel(const float* __restrict__ a, int K, uint4* hi, uint4* lo,
+                                                           _Float16* sh, _Float16* sl, float* __restrict__ inv, int* cnt, int ncnt) {
 #pragma clang fp contract(off)
-  __shared__ float red[8];
-  const int r = blockIdx.x, nb = K / 32;
-  const float* x = a + (size_t)r * K;
-  auto bsum = [&](int b) {
-    const float4* p = reinterpret_cast<const float4*>(x + 32 * b);
+  __shared__ float red[4];
+  if (blockIdx.x == 0)
+    for (int i = threadIdx.x; i < ncnt; i += 256) cnt[i] = 0;
+  const int r = blockIdx.x, n8 = K / 8, kb = K / 32;
+  const float4* x = reinterpret_cast<const float4*>(a + (size_t)r * K);
+  // the per-32 sum of the four chunks of this group of four lanes (eight float4 partials, left to
+  // right), in every lane of the group
+  auto bsum = [&](float4 p, float4 q) {
+    const float pa = (p.x + p.y) + (p.z + p.w), pb = (q.x + q.y) + (q.z + q.w);
     float s = 0.f;
 #pragma unroll
-    for (int t = 0; t < 8; ++t) {
-      const float4 v = p[t];
-      s += (v.x + v.y) + (v.z + v.w);
+    for (int t = 0; t < 4; ++t) {
+      s += __shfl(pa, (threadIdx.x & 60) + t, 64);
+      s += __shfl(pb, (threadIdx.x & 60) + t, 64);
     }
     return s;
   };
+  auto mag = [](float4 p) { return fmaxf(fmaxf(fabsf(p.x), fabsf(p.y)), fmaxf(fabsf(p.z), fabsf(p.w))); };
+  float4 xv[CPT][2];
   float m = 0.f;
-  for (int b = threadIdx.x; b < nb; b += 256) {
-    const float4* p = reinterpret_cast<const float4*>(x + 32 * b);
 #pragma unroll
-    for (int t = 0; t < 8; ++t) {
-      const float4 v = p[t];
-      m = fmaxf(m, fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))));
-    }
-    m = fmaxf(m, fabsf(bsum(b)));
+  for (int k = 0; k < CPT; ++k) {
+    const int e = 256 * k + (int)threadIdx.x, c = e < n8 ? e : 0;  // n8 % 4 == 0: a group is in or out together
+    xv[k][0] = x[2 * c];
+    xv[k][1] = x[2 * c + 1];
+    const float s = bsum(xv[k][0], xv[k][1]);
+    if (e < n8) m = fmaxf(m, fmaxf(fmaxf(mag(xv[k][0]), mag(xv[k][1])), fabsf(s)));
+  }
+  for (int e0 = 256 * CPT; e0 < n8; e0 += 256) {
+    const int e = e0 + (int)threadIdx.x, c = e < n8 ? e : 0;
+    const float4 p = x[2 * c], q = x[2 * c + 1];
+    const float s = bsum(p, q);
+    if (e < n8) m = fmaxf(m, fmaxf(fmaxf(mag(p), mag(q)), fabsf(s)));
   }
   m = wave_max(m);
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
@@ -299,29 +315,28 @@ __global__ __launch_bounds__(256) void split_scaled_kernel(const float* __restri
     scale = __uint_as_float((uint32_t)(127 + 14 - e) << 23);
   }
   if (threadIdx.x == 0) inv[r] = 1.f / scale;
-  for (int i = threadIdx.x; i < K; i += 256) {
-    const float v = x[i] * scale;
-    const _Float16 h = (_Float16)v;
-    hi[(size_t)r * K + i] = h;
-    lo[(size_t)r * K + i] = (_Float16)(v - (float)h);
+  // (a power-of-two factor commutes with the sums' roundings)
+  auto emit = [&](int e, float4 p, float4 q) {
+    const float v[8] = {p.x * scale, p.y * scale, p.z * scale, p.w * scale,
+                        q.x * scale, q.y * scale, q.z * scale, q.w * scale};
+    emit_split8(v, r, e < n8 ? e : 0, kb, e < n8, hi, lo, sh, sl, nullptr);
+  };
+#pragma unroll
+  for (int k = 0; k < CPT; ++k) emit(256 * k + (int)threadIdx.x, xv[k][0], xv[k][1]);
+  for (int e0 = 256 * CPT; e0 < n8; e0 += 256) {
+    const int e = e0 + (int)threadIdx.x, c = e < n8 ? e : 0;
+    emit(e, x[2 * c], x[2 * c + 1]);
   }
-  for (int b = threadIdx.x; b < nb; b += 256) {
-    const float v = bsum(b) * scale;
-    const _Float16 h = (_Float16)v;
-    sh[(size_t)r * nb + b] = h;
-    sl[(size_t)r * nb + b] = (_Float16)(v - (float)h);
-  }
-  (void)nb_total;
 }
 
-void launch_split_scaled(const float* a, int rows, int K, __half* hi, __half* lo, float* sums, float* inv,
-                         hipStream_t st) {
+void launch_split_scaled(const float* a, int rows, int K, __half* hi, __half* lo, float* sums, float* inv, int* cnt,
+                         int ncnt, hipStream_t st) {
   if (rows <= 0) return;
   if (K % 32 != 0 || reinterpret_cast<uintptr_t>(a) % 16) fail(ST_OP, "split_scaled: K % 32 and 16-byte aligned rows");
   const size_t nb = (size_t)rows * (K / 32);
   _Float16* s = reinterpret_cast<_Float16*>(sums);
-  hipLaunchKernelGGL(split_scaled_kernel, dim3(rows), dim3(256), 0, st, a, K, reinterpret_cast<_Float16*>(hi),
-                     reinterpret_cast<_Float16*>(lo), s, s + nb, nb, inv);
+  hipLaunchKernelGGL(split_scaled_kernel<8>, dim3(rows), dim3(256), 0, st, a, K, (uint4*)hi, (uint4*)lo, s, s + nb,
+                     inv, cnt, cnt ? ncnt : 0);
 }
 
 __global__ void row_scale_kernel(float* __restrict__ out, int N, const float* __restrict__ inv) {
@@ -441,7 +456,7 @@ void launch_swiglu(const float* g, const float* u, float* out, size_t n, hipStre
 // swiglu (as swiglu_kernel) over a [rows, K] input that also emits the GEMM input planes (the f32
 // output itself only when `out` is set).
 __global__ __launch_bounds__(256) void swiglu_split_kernel(const float* __restrict__ g, const float* __restrict__ u,
-                                                           float* __restrict__ out, size_t n8, uint4* hi, uint4* lo,
+                                                           float* __restrict__ out, size_t n8, uint32_t k8n, uint4* hi, uint4* lo,
                                                            _Float16* sh, _Float16* sl, int* ovf) {
 #pragma clang fp contract(off)
   for (size_t i0 = (size_t)blockIdx.x * 256; i0 < n8; i0 += (size_t)gridDim.x * 256) {
@@ -470,7 +485,7 @@ __global__ __launch_bounds__(256) void swiglu_split_kernel(const float* __restri
       reinterpret_cast<float4*>(out)[2 * c] = make_float4(v[0], v[1], v[2], v[3]);
       reinterpret_cast<float4*>(out)[2 * c + 1] = make_float4(v[4], v[5], v[6], v[7]);
     }
-    emit_split8(v, c, live, hi, lo, sh, sl, ovf);
+    emit_split8(v, (int)(c / k8n), (int)(c % k8n), k8n / 4, live, hi, lo, sh, sl, ovf);
   }
 }
 
@@ -482,8 +497,8 @@ void launch_swiglu_split(const float* g, const float* u, float* out, int rows, i
   const size_t n8 = (size_t)rows * (K / 8), nb = n8 / 4;
   _Float16* s = reinterpret_cast<_Float16*>(sums);
   const int blocks = (int)std::min<size_t>((n8 + 255) / 256, 4096);
-  hipLaunchKernelGGL(swiglu_split_kernel, dim3(blocks), dim3(256), 0, st, g, u, out, n8, (uint4*)hi, (uint4*)lo, s,
-                     s + nb, ovf);
+  hipLaunchKernelGGL(swiglu_split_kernel, dim3(blocks), dim3(256), 0, st, g, u, out, n8, (uint32_t)(K / 8), (uint4*)hi,
+                     (uint4*)lo, s, s + nb, ovf);
 }
 
 // gelu_tanh(g) * u (src/layers/ffn.rs:49-53); gelu_tanh_dev is in common.cuh.

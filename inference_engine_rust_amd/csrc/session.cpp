@@ -162,7 +162,7 @@ Session::~Session() {
                   (void*)d_flag_, (void*)d_cnt_, (void*)xs_, (void*)xsum_, kv_blob_, (void*)ple_tok_,
                   (void*)ple_proj_, (void*)ple_pack_, (void*)ple_tokd_, (void*)ple_projd_, (void*)ple_packd_,
                   (void*)xdec2_, (void*)xdec_save_, chain_blob_, (void*)d_chain_cnt_, (void*)d_chain_err_,
-                  (void*)d_ovf_, (void*)x_save_})
+                  (void*)d_ovf_, (void*)x_save_, (void*)sk_.cnt})
     dev_free(p);
   if (h_ovf_) (void)hipHostFree(h_ovf_);
   if (st_) (void)hipStreamDestroy(st_);
@@ -192,7 +192,18 @@ void Session::reset() {
 }
 
 void Session::ensure_rows(int rows) {
+  if (rows > 1 && sk_part_floats(rows) > sk_floats_) {  // K-split scratch of a few-row prefill
+    sync();
+    dev_free(sk_.cnt);
+    sk_.cnt = nullptr;
+    sk_floats_ = 0;
+    sk_.cnt = dev_alloc<int>(SK_MAX_GROUPS + sk_part_floats(rows));
+    sk_.part = reinterpret_cast<float*>(sk_.cnt + SK_MAX_GROUPS);
+    sk_floats_ = sk_part_floats(rows);
+    launch_fill_i32(sk_.cnt, 0, SK_MAX_GROUPS, st_);
+  }
   if (rows <= rows_cap_) return;
+  rows = (rows + 15) / 16 * 16;  // whole row tiles of the GEMM input planes
   sync();
   for (float** b : {&x_, &xn_, &q_, &k_, &v_, &att_, &g_, &u_, &act_, &tmp_, &ple_tok_, &ple_proj_, &ple_pack_}) {
     dev_free(*b);
@@ -259,7 +270,7 @@ static void project(const DevTensor& w, const float* a, const __half* xs, int ro
   } else if (f32) {
     launch_gemm_f32(w.dtype, w.dev, a, rows, K, N, out, resid, st);
   } else if (xs && gemm_mfma_ok(w.dtype, w.dev, K, N)) {
-    launch_gemm_mfma(w.dtype, w.dev, xs, xs + (size_t)rows * K, rows, K, N, out, resid, st);
+    launch_gemm_mfma(w.dtype, w.dev, xs, xs + plane_halves(rows, K), rows, K, N, out, resid, st);
   } else {
     launch_gemm(w.dtype, w.dev, a, rows, K, N, out, resid, st);
   }
@@ -317,8 +328,8 @@ bool Session::project_q(const DevTensor* const* ws, float* const* outs, int nseg
     segs[i] = GemmQSeg{p, outs[i], (int)w.dims[1]};
   }
   const __half* xh = xin ? xin : xs_;
-  const bool left = launch_gemm_q(dt, segs, nseg, xh, xh + (size_t)M * K, sin ? sin : xsum_, M, K, resid, st_, kpart,
-                                  pending != nullptr);
+  const bool left = launch_gemm_q(dt, segs, nseg, xh, xh + plane_halves(M, K), sin ? sin : xsum_, M, K, resid, st_, kpart,
+                                  pending != nullptr, nullptr, &sk_);
   if (pending) *pending = left;
   return true;
 }
@@ -339,8 +350,8 @@ bool Session::gate_up_glu(int li, int M) {
   if (dg != du) return false;
   const DevTensor* wd[1] = {&L.down};
   __half* ah = reinterpret_cast<__half*>(g_);
-  return launch_gemm_q_glu(dg, pg, pu, ffn, xs_, xs_ + (size_t)M * H_, xsum_, M, H_, ah, ah + (size_t)M * ffn, u_,
-                           quant_ready(wd, 1, M, ffn) ? nullptr : act_, d_ovf_, st_);
+  return launch_gemm_q_glu(dg, pg, pu, ffn, xs_, xs_ + plane_halves(M, H_), xsum_, M, H_, ah, ah + plane_halves(M, ffn), u_,
+                           quant_ready(wd, 1, M, ffn) ? nullptr : act_, d_ovf_, st_, &sk_);
 }
 
 bool Session::layer_prefill(int li, int M, bool pend_in) {
@@ -358,7 +369,7 @@ bool Session::layer_prefill(int li, int M, bool pend_in) {
   const bool f32 = f32_prefill_;
   auto split = [&](const float* a, int K) -> const __half* {
     if (!wide || K % 32 != 0) return nullptr;
-    launch_split_sums(a, M, K, xs_, xs_ + (size_t)M * K, xsum_, d_ovf_, st_);
+    launch_split_sums(a, M, K, xs_, xs_ + plane_halves(M, K), xsum_, d_ovf_, st_);
     return xs_;
   };
   // (the f32 output is written only when a consumer may fall back to it). A split-K partial left
@@ -369,7 +380,7 @@ bool Session::layer_prefill(int li, int M, bool pend_in) {
       launch_rmsnorm(x_, (const float*)w.dev, M, H_, eps, xn_, st_);
       return nullptr;
     }
-    launch_rmsnorm_split(x_, (const float*)w.dev, M, H_, eps, need_f32 ? xn_ : nullptr, xs_, xs_ + (size_t)M * H_,
+    launch_rmsnorm_split(x_, (const float*)w.dev, M, H_, eps, need_f32 ? xn_ : nullptr, xs_, xs_ + plane_halves(M, H_),
                          xsum_, d_ovf_, st_, pend ? tmp_ : nullptr);
     return xs_;
   };
@@ -444,7 +455,7 @@ bool Session::layer_prefill(int li, int M, bool pend_in) {
     if (wide && S.ffn_dim % 32 == 0) {
       const DevTensor* wd[1] = {&L.down};
       launch_swiglu_split(g_, u_, quant_ready(wd, 1, M, S.ffn_dim) ? nullptr : act_, M, S.ffn_dim, xs_,
-                          xs_ + (size_t)M * S.ffn_dim, xsum_, d_ovf_, st_);
+                          xs_ + plane_halves(M, S.ffn_dim), xsum_, d_ovf_, st_);
       xa = xs_;
     } else {
       launch_swiglu(g_, u_, act_, (size_t)M * S.ffn_dim, st_);
@@ -838,7 +849,7 @@ void Session::layer_decode_unfused(int li) {
 // the split takes; null otherwise.
 const __half* Session::split_rows(const float* a, int M, int K) {
   if (M < 2 || K % 32 != 0 || f32_prefill_) return nullptr;
-  launch_split_sums(a, M, K, xs_, xs_ + (size_t)M * K, xsum_, d_ovf_, st_);
+  launch_split_sums(a, M, K, xs_, xs_ + plane_halves(M, K), xsum_, d_ovf_, st_);
   return xs_;
 }
 
@@ -936,10 +947,16 @@ void Session::layer_prefill_gemma(int li, int M) {
     if (!L.ple_gate.present() || !L.ple_proj.present() || !L.ple_post_norm.present())
       fail(ST_MODEL, "PLE: missing inp_gate / proj / post_norm");
     xs = split_rows(x_, M, H_);
-    project(L.ple_gate, x_, xs, M, H_, pd, g_, nullptr, st_, f32_prefill_);
+    auto proj1 = [&](const DevTensor& w, const float* a, const __half* s, int K, int N, float* out) {
+      const DevTensor* ws[1] = {&w};
+      float* outs[1] = {out};
+      if (!s || w.dims.size() != 2 || (int)w.dims[1] != N || !project_q(ws, outs, 1, M, K, nullptr))
+        project(w, a, s, M, K, N, out, nullptr, st_, f32_prefill_);
+    };
+    proj1(L.ple_gate, x_, xs, H_, pd, g_);
     launch_ple_gate(g_, ple_pack_, M, pd, c.n_layers, li, st_);
     const __half* xg = split_rows(g_, M, pd);
-    project(L.ple_proj, g_, xg, M, pd, H_, tmp_, nullptr, st_, f32_prefill_);
+    proj1(L.ple_proj, g_, xg, pd, H_, tmp_);
     launch_rmsnorm_add(x_, tmp_, (const float*)L.ple_post_norm.dev, M, H_, eps, L.has_out_scale, L.out_scale_value,
                        st_);
   }

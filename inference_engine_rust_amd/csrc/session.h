@@ -112,6 +112,8 @@ class Session {
   __half* xs_ = nullptr;  // fp16 (hi, lo) split of the current prefill GEMM input
   size_t xs_halves_ = 0;
   size_t xs_halves() const { return xs_halves_; }
+  SkScratch sk_{nullptr, nullptr};  // K-split scratch of the few-row GEMM (one allocation, at cnt)
+  size_t sk_floats_ = 0;
   float* xsum_ = nullptr;  // its per-32 row sums (Q4_K min term)
   float *xdec_ = nullptr, *xdec2_ = nullptr, *xdec_save_ = nullptr, *xndec_ = nullptr, *qd_ = nullptr, *kd_ = nullptr, *vd_ = nullptr, *attd_ = nullptr;
   float *actd_ = nullptr, *logits_ = nullptr, *part_ = nullptr, *tmpd_ = nullptr;

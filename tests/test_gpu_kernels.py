@@ -142,6 +142,24 @@ def test_gemm_parity_mistral_shapes_m512(gpu, dt, k, n):
     _check_matmul(dt, k, n, 512)
 
 
+@pytest.mark.parametrize("dt,k,n,m", [
+    # few-row kernel: the packed-plane tile (up to 8 rows), one, two and four row tiles and their edges
+    *[(E.Q4K, 1024, 100, m) for m in (2, 8, 9, 16, 17, 32, 33, 64)],
+    # one superblock (a K wave without units), odd counts, K split over workgroups, ragged columns
+    (E.Q4K, 256, 64, 7), (E.Q4K, 768, 65, 12), (E.Q4K, 4096, 1024, 3), (E.Q6K, 256, 30, 5), (E.Q6K, 1280, 129, 20),
+    (E.Q6K, 4096, 200, 64), (E.Q6K, 14336, 64, 40), (E.Q6K, 2048, 300, 130),
+    # Q8_0: partial last unit (K % 256), the tensor's last bytes, two row-tile passes
+    (E.Q8_0, 32, 40, 2), (E.Q8_0, 288, 33, 8), (E.Q8_0, 1408, 70, 31), (E.Q8_0, 1536, 256, 50), (E.Q8_0, 6144, 96, 100),
+])
+def test_gemm_few_rows(gpu, dt, k, n, m):
+    _check_matmul(dt, k, n, m, seed=5)
+
+
+@pytest.mark.parametrize("dt,k,n,m", [(E.Q4K, 4096, 1024, 7), (E.Q6K, 1024, 130, 24), (E.Q8_0, 1408, 64, 40)])
+def test_gemm_few_rows_full_f32_range(gpu, dt, k, n, m):
+    _check_matmul(dt, k, n, m, seed=6, a=_wide_range_rows(m, k, 60 + dt))
+
+
 def _wide_range_rows(m, k, seed):
     """Activations over the f32 range the reference takes (src/ops/matmul.rs:176-204 multiplies any
     finite f32): row r is N(0, 1) scaled by 10^(-3 + 9 r / (m - 1)), up to 1e6; every 8th row also

@@ -133,9 +133,10 @@ void launch_split_sums(const float* a, int rows, int K, __half* hi, __half* lo, 
                        hipStream_t st);
 void launch_swiglu_split(const float* g, const float* u, float* out, int rows, int K, __half* hi, __half* lo,
                          float* sums, int* ovf, hipStream_t st);
-// *ovf = 1 when some |a[i]| (i < n) exceeds F16_PAIR_MAX (a prefill attention input the matrix-core
-// kernels split into fp16 pairs themselves).
-void launch_range_flag(const float* a, size_t n, int* ovf, hipStream_t st);
+// *ovf = 1 when some |value| of a (na of them), b or c (nbc each) exceeds F16_PAIR_MAX (prefill
+// attention inputs the matrix-core kernel splits into fp16 pairs itself).
+void launch_range_flag3(const float* a, size_t na, const float* b, const float* c, size_t nbc, int* ovf,
+                        hipStream_t st);
 // Op-level GEMM inputs with any f32 range: per row, the power-of-two factor s (1 unless the row's
 // largest |value| or per-32 sum exceeds 2^15, then the factor that brings it into [2^14, 2^15)),
 // the fp16 (hi, lo) planes of s * a and the per-32 sums of s * a (fp16 pair planes), and

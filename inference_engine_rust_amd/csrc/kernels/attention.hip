@@ -270,36 +270,44 @@ __global__ __launch_bounds__(256) void attn_prefill_mfma_kernel(const float* __r
 __global__ __launch_bounds__(256) void kv_split_kernel(const float* __restrict__ k, const float* __restrict__ v, int M,
                                                        int n_kv, int hd, int Mp, _Float16* __restrict__ kh,
                                                        _Float16* __restrict__ kl, _Float16* __restrict__ vh,
-                                                       _Float16* __restrict__ vl) {
+                                                       _Float16* __restrict__ vl, int* __restrict__ ovf) {
   __shared__ float tile[64][65];
   const int h = blockIdx.z, d0 = blockIdx.y * 64, p0 = blockIdx.x * 64, tid = threadIdx.x;
+  const int c4 = 4 * (tid & 15), d = d0 + c4;  // the thread's four head dims (hd is a multiple of 64)
   const size_t kvd = (size_t)n_kv * hd;
-#pragma unroll 4
-  for (int r = 0; r < 16; ++r) {
-    const int pl = (tid >> 6) + 4 * r, dl = tid & 63, p = p0 + pl, d = d0 + dl;
-    float vv = 0.f;
-    if (p < M && d < hd) {
+  bool big = false;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int pl = (tid >> 4) + 16 * r, p = p0 + pl;
+    float vv[4] = {0.f, 0.f, 0.f, 0.f};
+    if (p < M) {
       const size_t src = (size_t)p * kvd + (size_t)h * hd + d;
-      vv = v[src];
-      _Float16 a, b;
-      asplit(k[src], a, b);
+      _Float16 a[4], b[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float kx = k[src + i];
+        vv[i] = v[src + i];
+        big |= fmaxf(fabsf(kx), fabsf(vv[i])) > F16_PAIR_MAX;
+        asplit(kx, a[i], b[i]);
+      }
       const size_t kd = ((size_t)h * M + p) * hd + d;
-      kh[kd] = a;
-      kl[kd] = b;
+      *reinterpret_cast<uint2*>(kh + kd) = make_uint2(apack2(a[0], a[1]), apack2(a[2], a[3]));
+      *reinterpret_cast<uint2*>(kl + kd) = make_uint2(apack2(b[0], b[1]), apack2(b[2], b[3]));
     }
-    tile[pl][dl] = vv;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) tile[pl][c4 + i] = vv[i];
   }
+  if (big && ovf) *ovf = 1;
   __syncthreads();
-#pragma unroll 4
-  for (int r = 0; r < 16; ++r) {
-    const int dl = (tid >> 6) + 4 * r, pl = tid & 63, d = d0 + dl, p = p0 + pl;
-    if (d < hd && p < Mp) {
-      _Float16 a, b;
-      asplit(tile[pl][dl], a, b);
-      const size_t vd = ((size_t)h * hd + d) * Mp + p;
-      vh[vd] = a;
-      vl[vd] = b;
-    }
+#pragma unroll
+  for (int r = 0; r < 8; ++r) {
+    const int dl = (tid >> 5) + 8 * r, pl = 2 * (tid & 31);  // Mp is a multiple of 64: every p < Mp
+    _Float16 a[2], b[2];
+    asplit(tile[pl][dl], a[0], b[0]);
+    asplit(tile[pl + 1][dl], a[1], b[1]);
+    const size_t vd = ((size_t)h * hd + d0 + dl) * Mp + p0 + pl;
+    *reinterpret_cast<uint32_t*>(vh + vd) = apack2(a[0], a[1]);
+    *reinterpret_cast<uint32_t*>(vl + vd) = apack2(b[0], b[1]);
   }
 }
 
@@ -426,14 +434,19 @@ __global__ __launch_bounds__(256) void attn_prep_kernel(float* __restrict__ q, c
 // registers (no LDS round trip, no wave barrier), and 72 KB of LDS lets two workgroups share a
 // CU (NW = 4) or gives eight waves one staged block (NW = 8). Every product takes three MFMAs (hi*hi + hi*lo + lo*hi of the fp16 pairs, exact in f32);
 // the softmax is the online form per query. The longest (latest) query tiles are dispatched first.
-template <int HD, int TMQ, int NW, int KB>
-__global__ __launch_bounds__(64 * NW, 8 / NW) void attn_prefill_gqa_kernel(const float* __restrict__ q,
+// KG = 2: two sets of NW waves take the tile's key blocks in turn, each with its own staged block,
+// and the second set's (max, sum, O) are folded in through LDS at the end (head_dim 256, whose
+// grids leave most CUs idle: 800 rows of 8 query heads are 100 workgroups). `ovf` (when q was not
+// checked before): set when a q value is beyond the fp16 pair's range.
+template <int HD, int TMQ, int NW, int KB, int KG = 1>
+__global__ __launch_bounds__(64 * NW * KG, 8 / (NW * KG) > 0 ? 8 / (NW * KG) : 1) void attn_prefill_gqa_kernel(const float* __restrict__ q,
                                                                   const _Float16* __restrict__ kh,
                                                                   const _Float16* __restrict__ kl,
                                                                   const _Float16* __restrict__ vh,
                                                                   const _Float16* __restrict__ vl,
                                                                   float* __restrict__ out, int M, int Mp, int n_heads,
-                                                                  int n_kv, int window, float scale) {
+                                                                  int n_kv, int window, float scale,
+                                                                  int* __restrict__ ovf) {
   static_assert(KB == 32 || KB == 64, "keys per block");
   constexpr int JN = KB / 16;    // 16-key row tiles of S^T
   constexpr int KS = HD / 32;    // MFMA K steps of S^T
@@ -444,15 +457,20 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_prefill_gqa_kernel(const
   constexpr int NT = 64 * NW;
   constexpr int CPT = KB * HD / 8 / NT;  // 16-byte chunks per thread per plane of a K (or V^T) block
   static_assert(CPT >= 1 && (KB * HD / 8) % NT == 0, "block must divide over the threads");
-  __shared__ __align__(16) _Float16 ksh[KB][KROW];
-  __shared__ __align__(16) _Float16 ksl[KB][KROW];
-  __shared__ __align__(16) _Float16 vsh[HD][VROW];
-  __shared__ __align__(16) _Float16 vsl[HD][VROW];
+  struct Block {
+    _Float16 kh[KB][KROW], kl[KB][KROW], vh[HD][VROW], vl[HD][VROW];
+  };
+  __shared__ __align__(16) Block blk[KG];
 
   const int G = n_heads / n_kv, G4 = min(G, 4), HG = (G + 3) / 4;
   const int kvh = blockIdx.x / HG, hg = blockIdx.x % HG;
-  const int tid = threadIdx.x, lane = tid & 63;
+  const int kg = KG == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / NT);
+  const int tid = KG == 1 ? threadIdx.x : threadIdx.x % NT, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  auto& ksh = blk[kg].kh;
+  auto& ksl = blk[kg].kl;
+  auto& vsh = blk[kg].vh;
+  auto& vsl = blk[kg].vl;
   const int hl = wave % G4, qs = wave / G4, h = 4 * hg + hl;
   const bool active = h < G && qs < NW / G4;
   const int QT = QW * (NW / G4);
@@ -468,6 +486,7 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_prefill_gqa_kernel(const
   // (the softmax below is exp2(s - max), the same function), split into fp16 pairs
   const float qscale = scale * 1.44269504088896341f;
   au4_t qah[TMQ][KS], qal[TMQ][KS];
+  bool qbig = false;
 #pragma unroll
   for (int i = 0; i < TMQ; ++i) {
     const float* qrow = q + (size_t)min(q0 + 16 * i + fr, M - 1) * qd + (size_t)hq * HD;
@@ -477,6 +496,9 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_prefill_gqa_kernel(const
       const float4 b = *reinterpret_cast<const float4*>(qrow + 32 * s + fk + 4);
       const float vv[8] = {a.x * qscale, a.y * qscale, a.z * qscale, a.w * qscale,
                            b.x * qscale, b.y * qscale, b.z * qscale, b.w * qscale};
+      if (ovf)
+        qbig |= fmaxf(fmaxf(fmaxf(fabsf(a.x), fabsf(a.y)), fmaxf(fabsf(a.z), fabsf(a.w))),
+                      fmaxf(fmaxf(fabsf(b.x), fabsf(b.y)), fmaxf(fabsf(b.z), fabsf(b.w)))) > F16_PAIR_MAX;
       _Float16 hh[8], ll[8];
 #pragma unroll
       for (int t = 0; t < 8; ++t) asplit(vv[t], hh[t], ll[t]);
@@ -484,6 +506,7 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_prefill_gqa_kernel(const
       qal[i][s] = au4_t{apack2(ll[0], ll[1]), apack2(ll[2], ll[3]), apack2(ll[4], ll[5]), apack2(ll[6], ll[7])};
     }
   }
+  if (ovf && qbig) *ovf = 1;
   // O^T accumulators (lane: query fr, dims 16j + 4lg .. + 3) and the lane's query's softmax state
   // (running max in base-2 units, running sum)
   af4_t o[TMQ][NS];
@@ -520,8 +543,9 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_prefill_gqa_kernel(const
     }
   };
   const int kb_start = window > 0 ? (max(0, wq0 - (window - 1)) / KB) * KB : 0;
-  fetch(kb_start);
-  for (int kb0 = kb_start; kb0 <= wq1; kb0 += KB) {
+  fetch(min(kb_start + KB * kg, Mp - KB));
+  for (int kb1 = kb_start; kb1 <= wq1; kb1 += KB * KG) {
+    const int kb0 = kb1 + KB * kg;  // (the last round may leave the second set without a block)
     __syncthreads();  // the previous block's LDS reads are done
 #pragma unroll
     for (int c = 0; c < CPT; ++c) {
@@ -534,9 +558,9 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_prefill_gqa_kernel(const
       *reinterpret_cast<au4_t*>(&vsl[d][8 * vc]) = rv[1][c];
     }
     __syncthreads();
-    if (kb0 + KB <= wq1) fetch(kb0 + KB);
+    if (kb0 + KB * KG <= wq1) fetch(kb0 + KB * KG);
     // the wave's queries all precede the block, or the block is older than all their windows
-    if (!active || kb0 > q0 + QW - 1 || (window > 0 && kb0 + KB - 1 < q0 - (window - 1))) continue;
+    if (!active || (KG > 1 && kb0 > wq1) || kb0 > q0 + QW - 1 || (window > 0 && kb0 + KB - 1 < q0 - (window - 1))) continue;
     // query tiles that reach into the block (uniform); each K and V^T fragment is read from LDS
     // once and serves all of them
     bool live[TMQ];
@@ -642,17 +666,51 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_prefill_gqa_kernel(const
         if (TMQ > 1) __builtin_amdgcn_sched_barrier(0);
       }
   }
+  if constexpr (KG == 2) {
+    static_assert(KG == 1 || (TMQ == 1 && sizeof(Block) >= (size_t)NW * 64 * 4 * (4 * NS + 2)), "hand-over fits a block");
+    // [wave][value][lane], in the first set's block
+    float* hand = reinterpret_cast<float*>(&blk[0]) + (size_t)wave * 64 * (4 * NS + 2) + lane;
+    __syncthreads();
+    if (kg == 1) {
+      hand[0] = mrow[0];
+      hand[64] = lrow[0];
+#pragma unroll
+      for (int j = 0; j < NS; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) hand[64 * (2 + 4 * j + r)] = o[0][j][r];
+    }
+    __syncthreads();
+    if (kg == 1) return;
+    const float m1 = hand[0], l1 = hand[64];
+    const float mn = fmaxf(mrow[0], m1);
+    const float w0 = mrow[0] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mrow[0] - mn);
+    const float w1 = m1 == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m1 - mn);
+    lrow[0] = lrow[0] * w0 + l1 * w1;
+#pragma unroll
+    for (int j = 0; j < NS; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) o[0][j][r] = o[0][j][r] * w0 + hand[64 * (2 + 4 * j + r)] * w1;
+  }
   if (!active) return;
 #pragma unroll
   for (int i = 0; i < TMQ; ++i) {
     const int qi = q0 + 16 * i + fr;
     if (qi < M) {
+      // o / l with one reciprocal per query: its rounding error is taken out of each quotient by the
+      // remainder (l is a sum of exponentials, 1 or more; a full division per value was ten
+      // instructions)
       const float l = lrow[i];
+      float rc = __builtin_amdgcn_rcpf(l);
+      rc = fmaf(fmaf(-l, rc, 1.f), rc, rc);
+      auto quot = [&](float x) {
+        const float y = x * rc;
+        return fmaf(fmaf(-y, l, x), rc, y);
+      };
 #pragma unroll
       for (int j = 0; j < NS; ++j) {
         const af4_t v = o[i][j];
         *reinterpret_cast<float4*>(out + (size_t)qi * qd + (size_t)hq * HD + 16 * j + 4 * lg) =
-            make_float4(v[0] / l, v[1] / l, v[2] / l, v[3] / l);
+            make_float4(quot(v[0]), quot(v[1]), quot(v[2]), quot(v[3]));
       }
     }
   }
@@ -765,12 +823,6 @@ void launch_attn_prefill(const float* q, const float* k, const float* v, float* 
                          int head_dim, int window, float scale, hipStream_t st, void* scratch, size_t scratch_halves,
                          bool planes_ready, int* ovf) {
   const int G = n_heads / n_kv;
-  if (!planes_ready && ovf) {
-    // the kernels below split q, k and v into fp16 pairs themselves (or through kv_split_kernel)
-    launch_range_flag(q, (size_t)M * n_heads * head_dim, ovf, st);
-    launch_range_flag(k, (size_t)M * n_kv * head_dim, ovf, st);
-    launch_range_flag(v, (size_t)M * n_kv * head_dim, ovf, st);
-  }
   if (attn_planes_ok(M, n_heads, n_kv, head_dim, scratch, scratch_halves) && G >= 1) {
     const int Mp = ((M + 63) / 64) * 64;
     const size_t plane = (size_t)n_kv * head_dim * Mp;
@@ -778,36 +830,37 @@ void launch_attn_prefill(const float* q, const float* k, const float* v, float* 
     _Float16 *kh = s16, *kl = s16 + plane, *vh = s16 + 2 * plane, *vl = s16 + 3 * plane;
     if (!planes_ready)
       hipLaunchKernelGGL(kv_split_kernel, dim3(Mp / 64, (head_dim + 63) / 64, n_kv), dim3(256), 0, st, k, v, M, n_kv,
-                         head_dim, Mp, kh, kl, vh, vl);
+                         head_dim, Mp, kh, kl, vh, vl, ovf);
+    int* qovf = planes_ready ? nullptr : ovf;
     const int G4 = std::min(G, 4), HG = (G + 3) / 4;
+    // query tile of NW waves of TMQ 16-query tiles each
+    auto tile = [&](int tmq, int nw) { return 16 * tmq * (nw / G4); };
+    auto wgs = [&](int qt) { return (size_t)n_kv * HG * ((M + qt - 1) / qt); };
+#define IEK_GQA(HD, TMQ, NW, KB, KG)                                                                                \
+  hipLaunchKernelGGL((attn_prefill_gqa_kernel<HD, TMQ, NW, KB, KG>),                                                \
+                     dim3(n_kv * HG, (M + tile(TMQ, NW) - 1) / tile(TMQ, NW)), dim3(64 * NW * KG), 0, st, q, kh, kl, \
+                     vh, vl, out, M, Mp, n_heads, n_kv, window, scale, qovf)
     // eight waves of two query tiles each per staged block once the grid fills the machine twice
-    // over, four waves of one tile below that
-    const int qt8 = 32 * (8 / G4);
-    const bool wide = (size_t)n_kv * HG * ((M + qt8 - 1) / qt8) >= 2 * (size_t)num_cus();
-    const int QT = wide ? qt8 : 16 * (4 / G4);
-    const dim3 grid(n_kv * HG, (M + QT - 1) / QT);
+    // over (4096 rows of 32 heads: 393 us against 510), four waves of one tile below that (2045
+    // rows: 146 against 176; four waves of two tiles 171)
+    const bool wide = wgs(tile(2, 8)) >= 2 * (size_t)num_cus();
     if (head_dim == 256) {
-      // 32-key blocks (the K and V^T planes of a block take 75 KB), four waves of one tile
-      const int qt4 = 16 * (4 / G4);
-      hipLaunchKernelGGL((attn_prefill_gqa_kernel<256, 1, 4, 32>), dim3(n_kv * HG, (M + qt4 - 1) / qt4), dim3(256), 0,
-                         st, q, kh, kl, vh, vl, out, M, Mp, n_heads, n_kv, window, scale);
+      // 32-key blocks (the K and V^T planes of a block take 75 KB); one set of four waves took 60 us
+      // for 800 rows of 8 heads and 66 us for 2045, two sets 50 and 55
+      IEK_GQA(256, 1, 4, 32, 2);
     } else if (head_dim == 128) {
-      if (wide)
-        hipLaunchKernelGGL((attn_prefill_gqa_kernel<128, 2, 8, 64>), grid, dim3(512), 0, st, q, kh, kl, vh, vl, out, M,
-                           Mp, n_heads, n_kv, window, scale);
-      else
-        hipLaunchKernelGGL((attn_prefill_gqa_kernel<128, 1, 4, 64>), grid, dim3(256), 0, st, q, kh, kl, vh, vl, out, M,
-                           Mp, n_heads, n_kv, window, scale);
+      if (wide) IEK_GQA(128, 2, 8, 64, 1);
+      else IEK_GQA(128, 1, 4, 64, 1);
     } else {
-      if (wide)
-        hipLaunchKernelGGL((attn_prefill_gqa_kernel<64, 2, 8, 64>), grid, dim3(512), 0, st, q, kh, kl, vh, vl, out, M,
-                           Mp, n_heads, n_kv, window, scale);
-      else
-        hipLaunchKernelGGL((attn_prefill_gqa_kernel<64, 1, 4, 64>), grid, dim3(256), 0, st, q, kh, kl, vh, vl, out, M,
-                           Mp, n_heads, n_kv, window, scale);
+      if (wide) IEK_GQA(64, 2, 8, 64, 1);
+      else IEK_GQA(64, 1, 4, 64, 1);
     }
+#undef IEK_GQA
     return;
   }
+  // the kernel below splits q, k and v into fp16 pairs itself
+  if (!planes_ready && ovf)
+    launch_range_flag3(q, (size_t)M * n_heads * head_dim, k, v, (size_t)M * n_kv * head_dim, ovf, st);
   dim3 grid(n_heads, (M + 63) / 64);
   switch (head_dim) {
 #define IEK_AP(HD, KB)                                                                                          \

@@ -245,19 +245,23 @@ void launch_split_sums(const float* a, int rows, int K, __half* hi, __half* lo, 
                      s + nb, ovf);
 }
 
-// *ovf = 1 when some |a[i]| exceeds the fp16 pair's range (NaN does not count: it stays NaN on
-// either path).
-__global__ __launch_bounds__(256) void range_flag_kernel(const float* __restrict__ a, size_t n, int* ovf) {
+// *ovf = 1 when a value of a, b or c exceeds the fp16 pair's range (NaN does not count: it stays
+// NaN on either path). Grid row y takes array y.
+__global__ __launch_bounds__(256) void range_flag3_kernel(const float* __restrict__ a, size_t na, const float* __restrict__ b,
+                                                          const float* __restrict__ c, size_t nbc, int* ovf) {
+  const float* x = blockIdx.y == 0 ? a : blockIdx.y == 1 ? b : c;
+  const size_t n = blockIdx.y == 0 ? na : nbc;
   bool big = false;
   for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256)
-    big |= fabsf(a[i]) > F16_PAIR_MAX;
+    big |= fabsf(x[i]) > F16_PAIR_MAX;
   if (big) *ovf = 1;
 }
 
-void launch_range_flag(const float* a, size_t n, int* ovf, hipStream_t st) {
-  if (n == 0 || !ovf) return;
-  const int blocks = (int)std::min<size_t>((n + 255) / 256, 2048);
-  hipLaunchKernelGGL(range_flag_kernel, dim3(blocks), dim3(256), 0, st, a, n, ovf);
+void launch_range_flag3(const float* a, size_t na, const float* b, const float* c, size_t nbc, int* ovf,
+                        hipStream_t st) {
+  if (na == 0 || !ovf) return;
+  const int blocks = (int)std::min<size_t>((std::max(na, nbc) + 255) / 256, 2048);
+  hipLaunchKernelGGL(range_flag3_kernel, dim3(blocks, 3), dim3(256), 0, st, a, na, b, c, nbc, ovf);
 }
 
 // Per-row scaled GEMM input (op level): one workgroup per row. Pass 1 finds the row's largest

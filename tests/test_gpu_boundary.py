@@ -224,6 +224,32 @@ def test_dev_attention_prefill_matches_oracle(gpu, n_heads, n_kv, hd, seq, windo
     assert worst < 1e-4, worst
 
 
+@pytest.mark.parametrize("n_heads,n_kv,seq,window", [(8, 1, 1, 0), (8, 1, 31, 0), (8, 1, 33, 0), (4, 2, 65, 16),
+                                                     (3, 1, 96, 33), (8, 8, 129, 0), (8, 1, 577, 512)])
+def test_dev_attention_prefill_key_sets(gpu, n_heads, n_kv, seq, window):
+    """head_dim 256: the two wave sets that take the key blocks in turn, at block edges (32 keys),
+    with an odd block count, a window that skips blocks and query groups that leave waves idle."""
+    test_dev_attention_prefill_matches_oracle(gpu, n_heads, n_kv, 256, seq, window)
+
+
+@pytest.mark.parametrize("which", [0, 1, 2])
+@pytest.mark.parametrize("hd", [64, 256, 512])
+def test_dev_attention_prefill_range_of_each_input(gpu, hd, which):
+    """One value past the fp16 pair's range in q, k or v alone (the last row's last dim) is seen by
+    the kernel that splits that input, and the f32 kernel's result comes back."""
+    n_heads, n_kv, seq = 4, 1, 70
+    rng = np.random.default_rng(hd + which)
+    x = [rng.standard_normal(seq * n * hd).astype(np.float32) for n in (n_heads, n_kv, n_kv)]
+    x[which][-1] = 1e5
+    scale = 1e-3
+    want = O.attention_prefill(*x, seq, n_heads, n_kv, hd, -1, scale)
+    d = [torch.from_numpy(a).to("cuda") for a in x]
+    out = torch.empty(seq * n_heads * hd, dtype=torch.float32, device="cuda")
+    E.attention_prefill(*(t.data_ptr() for t in d), seq, n_heads, n_kv, hd, 0, scale, out.data_ptr(),
+                        torch.cuda.current_stream().cuda_stream)
+    assert rel_l2(out.cpu().numpy(), want) < 1e-5
+
+
 def test_dev_attention_prefill_beyond_fp16_range_and_errors(gpu):
     """Scores from inputs past 65 504 (the fp16 pairs' range) take the f32 kernel: still the
     oracle's result; and the entry's errors."""

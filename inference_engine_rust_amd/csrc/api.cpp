@@ -305,7 +305,7 @@ static uint32_t argmax_dev(const float* logits, size_t n, unsigned long long* sc
   return host;
 }
 
-// Checks of the decode attention op; returns the partial-buffer floats it needs.
+// Checks of the decode attention op; returns the partial-buffer floats of a full cache.
 static size_t attention_check(size_t n_heads, size_t n_kv, size_t hd, size_t max_len, size_t total) {
   if (n_kv == 0 || n_heads == 0 || n_heads % n_kv != 0 || n_heads / n_kv > 8)
     fail(ST_OP, "attention: GQA group must divide the heads and be at most 8");
@@ -318,16 +318,15 @@ static size_t attention_check(size_t n_heads, size_t n_kv, size_t hd, size_t max
   return attn_decode_part_floats((int)n_heads, (int)hd, (int)max_len);
 }
 
-// counters (2 * n_kv ints) cleared and the position (total - 1) set by small kernels, so the
-// sequence is safe under stream capture; the kernel leaves the counters zero again.
+// counters (2 * n_kv ints) cleared by a small kernel, so the sequence is safe under stream capture;
+// the length goes by value, and the chunks are sized for it and not for the cache's capacity.
 static void attention_launch(const float* q, const void* kc, const void* vc, bool kv_f32, size_t n_heads, size_t n_kv,
                              size_t hd, size_t max_len, size_t total, size_t window, float scale, float* out,
-                             float* part, int* cnt, int* pos, hipStream_t st) {
+                             float* part, int* cnt, hipStream_t st) {
   const int win = window >= total ? 0 : (int)window;  // a window covering every key is no window
   launch_fill_i32(cnt, 0, 2 * (int)n_kv, st);
-  launch_set_int(pos, (int)(total - 1), st);
-  launch_attn_decode(q, kc, vc, kv_f32, out, part, cnt, (int)n_heads, (int)n_kv, (int)hd, (int)max_len, pos, win,
-                     scale, (int)max_len, st);
+  launch_attn_decode(q, kc, vc, kv_f32, out, part, cnt, (int)n_heads, (int)n_kv, (int)hd, (int)max_len, nullptr, win,
+                     scale, (int)total, st, (int)total);
   after_launch();
 }
 
@@ -448,15 +447,16 @@ iek_status iek_dev_attention_decode(const float* q, const void* k_cache, const v
                                     size_t total_pos, size_t sliding_window, float scale, float* out, void* stream) {
   IEK_API_TRY({
     if (kv_dtype != IEK_F16 && kv_dtype != IEK_F32) fail(ST_OP, "attention: KV cache dtype must be F16 or F32");
-    const size_t pf = attention_check(n_heads, n_kv_heads, head_dim, max_seq_len, total_pos);
+    attention_check(n_heads, n_kv_heads, head_dim, max_seq_len, total_pos);
+    const size_t pf = attn_decode_part_floats((int)n_heads, (int)head_dim, (int)total_pos);
     hipStream_t st = as_stream(stream);
     char* scratch = nullptr;
     const size_t cnt_off = (pf * 4 + 255) / 256 * 256;
-    IEK_HIP(hipMalloc(&scratch, cnt_off + (2 * n_kv_heads + 1) * 4));
+    IEK_HIP(hipMalloc(&scratch, cnt_off + 2 * n_kv_heads * 4));
     try {
       int* cnt = reinterpret_cast<int*>(scratch + cnt_off);
       attention_launch(q, k_cache, v_cache, kv_dtype == IEK_F32, n_heads, n_kv_heads, head_dim, max_seq_len, total_pos,
-                       sliding_window, scale, out, reinterpret_cast<float*>(scratch), cnt, cnt + 2 * n_kv_heads, st);
+                       sliding_window, scale, out, reinterpret_cast<float*>(scratch), cnt, st);
       IEK_HIP(hipStreamSynchronize(st));  // the scratch is freed below
     } catch (...) {
       (void)hipFree(scratch);
@@ -521,7 +521,7 @@ iek_status iek_dev_attention_decode_noalloc(const float* q, const void* k_cache,
     int* cnt = reinterpret_cast<int*>(base);
     float* part = reinterpret_cast<float*>(base + NOALLOC_COUNTER_BYTES);
     attention_launch(q, k_cache, v_cache, kv_dtype == IEK_F32, n_heads, n_kv_heads, head_dim, max_seq_len, total_pos,
-                     sliding_window, scale, out, part, cnt, cnt + 2 * n_kv_heads, as_stream(stream));
+                     sliding_window, scale, out, part, cnt, as_stream(stream));
   })
 }
 
@@ -728,13 +728,13 @@ iek_status iek_attention_decode(const float* q, const float* k_cache, const floa
         std::memcpy(&vt[dst], v_cache + src, head_dim * 4);
       }
     const size_t qn = n_heads * head_dim * 4;
-    HostCall hc({qn, kvn * 4, kvn * 4, qn, pf * 4, (2 * n_kv_heads + 1) * 4});
+    HostCall hc({qn, kvn * 4, kvn * 4, qn, pf * 4, 2 * n_kv_heads * 4});
     const float* dq = hc.up<float>(0, q, qn);
     const float* dk = hc.up<float>(1, kt.data(), kvn * 4);
     const float* dv = hc.up<float>(2, vt.data(), kvn * 4);
     int* cnt = hc.ptr<int>(5);
     attention_launch(dq, dk, dv, true, n_heads, n_kv_heads, head_dim, total_pos, total_pos, sliding_window, scale,
-                     hc.ptr<float>(3), hc.ptr<float>(4), cnt, cnt + 2 * n_kv_heads, hc.st);
+                     hc.ptr<float>(3), hc.ptr<float>(4), cnt, hc.st);
     hc.down(out, hc.ptr<float>(3), qn);
     hc.finish();
   })

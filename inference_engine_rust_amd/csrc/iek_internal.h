@@ -180,11 +180,12 @@ void launch_unpack_qk(const float* src, float* dst, int rows, int row_stride, in
 void launch_copy_f32(const float* src, float* dst, size_t n, hipStream_t st);
 void launch_fill_i32(int* p, int v, int n, hipStream_t st);
 // `counters` holds 2 * n_kv zero-initialised ints (one per KV head and query-head group); the
-// kernel leaves them zero again.
-// The cache is fp16, or f32 when kv_f32 (Gemma-4 sessions).
+// kernel leaves them zero again. The cache is fp16, or f32 when kv_f32. pos_dev: the position (keys
+// - 1) in device memory, the chunks sized for max_len keys; or null and `total` keys (max_len =
+// total).
 void launch_attn_decode(const float* q, const void* kc, const void* vc, bool kv_f32, float* out, float* part,
                         int* counters, int n_heads, int n_kv, int head_dim, int ctx, const int* pos_dev, int window,
-                        float scale, int max_len, hipStream_t st);
+                        float scale, int max_len, hipStream_t st, int total = 0);
 // Floats of `part` that launch_attn_decode needs at most for a cache of max_len keys.
 size_t attn_decode_part_floats(int n_heads, int head_dim, int max_len);
 // The no-allocation scratch (kernels/noalloc.hip): a file-scope device array of this many bytes

@@ -1,13 +1,13 @@
 // Attention over a KV cache laid out per layer as [n_kv][ctx][head_dim] (f32 in the sessions; fp16
 // through the op-level entry).
 //
-// Decode (src/layers/attention.rs:462-655): split-K flash-decode over 64-key slices, GQA groups
-// sharing one K/V stream; the slice count is fixed by the cache capacity so the launch shape
-// never changes between captured decode steps, and the live length is read from device memory.
+// Decode (src/layers/attention.rs:462-655): split-K flash-decode over chunks of keys, GQA groups
+// sharing one K/V stream; in a session the chunks are fixed by the cache capacity, so the launch
+// shape never changes between captured decode steps, and the live length is read from device memory.
 //
 // Prefill (attention.rs:175-422): causal attention over the f32 K/V of the prompt (the
 // reference attends to the layer's own k_data/v_data, not the cache).
-#include <cstdlib>
+#include <cmath>
 #include <type_traits>
 
 #include "attn_core.cuh"
@@ -19,78 +19,119 @@ __global__ __launch_bounds__(256 * SETS) void attn_decode_kernel(const float* __
                                                                  const T* __restrict__ vc, float* __restrict__ part,
                                                                  float* __restrict__ out, int* __restrict__ counters,
                                                                  int n_heads, int n_kv, int ctx, const int* pos_dev,
-                                                                 int window, float scale, int nsplit, int spc,
-                                                                 int HG) {
+                                                                 int total, int window, float scale, int nsplit,
+                                                                 int spc, int HG) {
   __shared__ __align__(16) char smem[AttnSmem<HD, SETS, T>::BYTES];
   // all arguments in one batch of scalar loads, ahead of the position they depend on
   asm volatile("" ::"s"(q), "s"(kc), "s"(vc), "s"(part), "s"(out), "s"(counters), "s"(n_heads), "s"(n_kv), "s"(ctx),
-               "s"(pos_dev), "s"(window), "s"(scale), "s"(nsplit), "s"(spc), "s"(HG));
-  attn_chunk<HD, COH, EARLY, SETS, T>(q, kc, vc, part, out, counters, n_heads, n_kv, ctx, pos_dev, 0, window, scale,
+               "s"(pos_dev), "s"(total), "s"(window), "s"(scale), "s"(nsplit), "s"(spc), "s"(HG));
+  attn_chunk<HD, COH, EARLY, SETS, T>(q, kc, vc, part, out, counters, n_heads, n_kv, ctx, pos_dev, total, window, scale,
                                       nsplit, blockIdx.x / HG, blockIdx.y, spc, smem, blockIdx.x % HG, HG);
 }
 
+// head_dim 256 and 512. Latency-bound: one launch reads under 2 MB at the contexts of the models with
+// such heads. Against slices of 64 keys staged in LDS (two workgroup barriers a slice, every head's
+// wave reading the whole slice back from LDS): 75 keys of one KV head 8.6 -> 6.8 us at 256, 14.8 ->
+// 9.5 at 512; 500 keys of 512 17.4 -> 11.8; 8000 keys 54 -> 28.
+template <int HD, bool EARLY, typename T>
+__global__ __launch_bounds__(256) void attn_decode_wide_kernel(const float* __restrict__ q, const T* __restrict__ kc,
+                                                               const T* __restrict__ vc, float* __restrict__ part,
+                                                               float* __restrict__ out, int* __restrict__ counters,
+                                                               int n_heads, int n_kv, int ctx, const int* pos_dev,
+                                                               int total, int window, float scale, int nslot, int CK,
+                                                               int HG) {
+  __shared__ __align__(16) AttnWide<HD> smem;
+  asm volatile("" ::"s"(q), "s"(kc), "s"(vc), "s"(part), "s"(out), "s"(counters), "s"(n_heads), "s"(n_kv), "s"(ctx),
+               "s"(pos_dev), "s"(total), "s"(window), "s"(scale), "s"(nslot), "s"(CK), "s"(HG));
+  attn_chunk_wide<HD, EARLY, T>(q, kc, vc, part, out, counters, n_heads, n_kv, ctx, pos_dev, total, window, scale,
+                                nslot, blockIdx.x / HG, blockIdx.y, CK, smem, blockIdx.x % HG, HG);
+}
+
 template <int HD, typename T>
-static void attn_decode_hd(dim3 grid, hipStream_t st, const float* q, const T* kc, const T* vc, float* out, float* part,
-                           int* counters, int n_heads, int n_kv, int ctx, const int* pos_dev, int window, float scale,
-                           int nsplit) {
+static void attn_decode_hd(hipStream_t st, const float* q, const T* kc, const T* vc, float* out, float* part,
+                           int* counters, int n_heads, int n_kv, int ctx, const int* pos_dev, int total, int window,
+                           float scale, int max_len) {
   // chunks of spc slices (about 32 chunks per KV head); one partial slot per chunk
-  const int spc = attn_slices_per_chunk(nsplit * SPLIT, window, 32);
-  const int nchunk = (nsplit + spc - 1) / spc;
-  // Chunks of several slices (long contexts) run two slice streams per workgroup (head dims up to
-  // 128: the doubled K / V buffers still fit in LDS), and publish their partials with coherent
-  // stores and a relaxed count (no L2 write-back / invalidate around the arrival, measured faster
-  // there; one-slice chunks are faster with plain stores).
-  const bool two = HD <= 128 && spc >= 2;
+  const int spc = attn_slices_per_chunk(max_len, window, 32);
+  const int nchunk = ((max_len + SPLIT - 1) / SPLIT + spc - 1) / spc;
+  // Chunks of several slices (long contexts) run two slice streams per workgroup, and publish their
+  // partials with coherent stores and a relaxed count (no L2 write-back / invalidate around the
+  // arrival, measured faster there; one-slice chunks are faster with plain stores).
+  const bool two = spc >= 2;
   // A group of 8 query heads splits over two workgroups per chunk (four heads each, one per
-  // wave) when there are few KV heads to spread over the machine (Gemma-4-E2B: one KV head);
+  // wave) when there are few KV heads to spread over the machine (one KV head: Gemma-4-E2B);
   // each half has its own arrival counter (2 * n_kv counters) and merge.
   const int HG = (n_heads / n_kv == 8 && n_kv < 4) ? 2 : 1;
   auto go = [&](auto kern, int nt) {
-    hipLaunchKernelGGL(kern, dim3(grid.x * HG, nchunk), dim3(nt), 0, st, q, kc, vc, part, out, counters, n_heads, n_kv,
-                       ctx, pos_dev, window, scale, nchunk, spc, HG);
+    hipLaunchKernelGGL(kern, dim3(n_kv * HG, nchunk), dim3(nt), 0, st, q, kc, vc, part, out, counters, n_heads, n_kv,
+                       ctx, pos_dev, total, window, scale, nchunk, spc, HG);
   };
   // without a window the first slice's loads go out before the position is known
-  constexpr int S2 = HD <= 128 ? 2 : 1;
   if (window <= 0)
-    two ? go(attn_decode_kernel<HD, true, S2, true, T>, 512) : go(attn_decode_kernel<HD, true, 1, false, T>, 256);
+    two ? go(attn_decode_kernel<HD, true, 2, true, T>, 512) : go(attn_decode_kernel<HD, true, 1, false, T>, 256);
   else
-    two ? go(attn_decode_kernel<HD, false, S2, true, T>, 512) : go(attn_decode_kernel<HD, false, 1, false, T>, 256);
+    two ? go(attn_decode_kernel<HD, false, 2, true, T>, 512) : go(attn_decode_kernel<HD, false, 1, false, T>, 256);
+}
+
+// Partial slots per query head: one per 64 keys; at head_dim 256 and up, whose chunks go down to 8
+// keys, one per 8 as far as that keeps n_heads * slots within 4096.
+static int attn_slots(int n_heads, int head_dim, int max_len) {
+  const int n = (max_len + SPLIT - 1) / SPLIT;
+  return head_dim < 256 ? n : std::max(n, std::min((max_len + 7) / 8, 4096 / std::max(n_heads, 1)));
+}
+
+template <int HD, typename T>
+static void attn_decode_wide(hipStream_t st, const float* q, const T* kc, const T* vc, float* out, float* part,
+                             int* counters, int n_heads, int n_kv, int ctx, const int* pos_dev, int total, int window,
+                             float scale, int max_len) {
+  const int HG = (n_heads / n_kv + 3) / 4;
+  // Keys per chunk: a chunk's time grows with its keys and the merge's with the number of chunks,
+  // so about sqrt(2 * keys) of them (a window keeps only ~window keys live). Measured with 16 / 32 /
+  // 64 chunks per KV head, one KV head of 512: 11.8 / 13.3 / 17.5 us at 500 keys, 20.2 / 17.3 / 19.9
+  // at 2000, 49 / 33 / 28 at 8000. In whole steps of the workgroup, within the partial slots.
+  constexpr int UNIT = AttnWide<HD>::UNIT;
+  const int span = window > 0 ? std::min(max_len, window) : max_len, slots = attn_slots(n_heads, HD, max_len);
+  const int keys = std::max((int)std::sqrt(2.0 * span), (max_len + slots - 1) / slots);
+  const int CK = (keys + UNIT - 1) / UNIT * UNIT, nchunk = (max_len + CK - 1) / CK;
+  auto go = [&](auto kern) {
+    hipLaunchKernelGGL(kern, dim3(n_kv * HG, nchunk), dim3(256), 0, st, q, kc, vc, part, out, counters, n_heads, n_kv,
+                       ctx, pos_dev, total, window, scale, nchunk, CK, HG);
+  };
+  // without a window the first step's loads go out before the position is known
+  window <= 0 ? go(attn_decode_wide_kernel<HD, true, T>) : go(attn_decode_wide_kernel<HD, false, T>);
 }
 
 size_t attn_decode_part_floats(int n_heads, int head_dim, int max_len) {
-  // one (max, sum, o[head_dim]) slot per query head and 64-key slice bounds both kernels' partials
-  return (size_t)n_heads * ((max_len + SPLIT - 1) / SPLIT) * (head_dim + 2);
+  return (size_t)n_heads * attn_slots(n_heads, head_dim, max_len) * (head_dim + 2);
 }
 
 void launch_attn_decode(const float* q, const void* kc, const void* vc, bool kv_f32, float* out, float* part,
                         int* counters, int n_heads, int n_kv, int head_dim, int ctx, const int* pos_dev, int window,
-                        float scale, int max_len, hipStream_t st) {
-  const int nsplit = (max_len + SPLIT - 1) / SPLIT;
-  dim3 grid(n_kv, nsplit);
+                        float scale, int max_len, hipStream_t st, int total) {
   if (n_kv <= 0 || n_heads % n_kv != 0 || n_heads / n_kv > 8)
     fail(ST_OP, "attention: GQA group must divide the heads and be at most 8");
+#define IEK_AD(FN, HD)                                                                                              \
+  kv_f32 ? FN<HD>(st, q, (const float*)kc, (const float*)vc, out, part, counters, n_heads, n_kv, ctx, pos_dev,      \
+                  total, window, scale, max_len)                                                                    \
+         : FN<HD>(st, q, (const __half*)kc, (const __half*)vc, out, part, counters, n_heads, n_kv, ctx, pos_dev,    \
+                  total, window, scale, max_len)
   switch (head_dim) {
-#define IEK_AD(HD)                                                                                                 \
-  kv_f32 ? attn_decode_hd<HD>(grid, st, q, (const float*)kc, (const float*)vc, out, part, counters, n_heads, n_kv, ctx, \
-                              pos_dev, window, scale, nsplit)                                                         \
-         : attn_decode_hd<HD>(grid, st, q, (const __half*)kc, (const __half*)vc, out, part, counters, n_heads, n_kv,   \
-                              ctx, pos_dev, window, scale, nsplit)
     case 64:
-      IEK_AD(64);
+      IEK_AD(attn_decode_hd, 64);
       break;
     case 128:
-      IEK_AD(128);
+      IEK_AD(attn_decode_hd, 128);
       break;
     case 256:
-      IEK_AD(256);
+      IEK_AD(attn_decode_wide, 256);
       break;
     case 512:
-      IEK_AD(512);
+      IEK_AD(attn_decode_wide, 512);
       break;
-#undef IEK_AD
     default:
       fail(ST_OP, "attention: head_dim must be 64, 128, 256 or 512");
   }
+#undef IEK_AD
 }
 
 // Prefill on the matrix cores (v_mfma_f32_16x16x32_f16): one 256-thread workgroup per (head,

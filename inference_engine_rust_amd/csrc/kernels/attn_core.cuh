@@ -87,8 +87,9 @@ IEK_DEV void merge_head(const float* __restrict__ part, float* __restrict__ out,
 // barrier orders every wave's partial stores before thread 0's agent-scope acq_rel add (which
 // writes back this XCD's L2); the last arrival's acquire side invalidates its L2 before the
 // partials are read. The counter is reset for the next launch.
-// s0 .. nlive-1 are the live partial slots of the KV head. WIDE: up to twice the batch when that
-// fetches the live slots in one round trip (many-slot merges).
+// s0 .. nlive-1 are the live partial slots of the KV head. WIDE: twice the batch when that fetches
+// the live slots in one round trip (many-slot merges), and at head_dim 256 and up, whose batches are
+// few rows, for all but the smallest.
 template <int HD, bool COH = false, bool WIDE = false>
 // The last workgroup to arrive on counters[cidx] merges query heads [gb, gb + gn) of KV head kvh
 // (G query heads per KV head).
@@ -114,7 +115,7 @@ IEK_DEV void merge_if_last(const float* __restrict__ part, float* __restrict__ o
   if (!last) return;
   if (!COH) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
   constexpr int B1 = HD >= 512 ? 4 : 2048 / HD;  // 32 floats per lane
-  const bool wide = WIDE && nlive - s0 > B1 && nlive - s0 <= 2 * B1;
+  const bool wide = WIDE && nlive - s0 > B1 && (HD >= 256 || nlive - s0 <= 2 * B1);
   for (int g = gb + wave; g < gb + gn; g += 4) {
     if (WIDE && wide)
       merge_head<HD, COH, 2 * B1>(part, out, kvh * G + g, nsplit, s0, nlive, wsl + 256 * wave);
@@ -123,15 +124,14 @@ IEK_DEV void merge_if_last(const float* __restrict__ part, float* __restrict__ o
   }
 }
 
-// LDS of one slice item: K rows (padded), V rows (HD <= 256), the group's q, the wave's
+// LDS of one slice item (head_dim up to 128): K rows (padded), V rows, the group's q, the wave's
 // probabilities, the merge weights and the last-arrival flag; K, V and the probabilities once per
 // slice stream (SETS).
 template <int HD, int SETS = 1, typename T = __half>
 struct AttnSmem {
   static constexpr int ES = (int)sizeof(T);
   static constexpr int KROW = HD + 16 / ES;  // padded K row: 16 bytes
-  static constexpr bool VL = HD <= 256;
-  static constexpr size_t KS1 = (size_t)SPLIT * KROW * ES, VS1 = VL ? (size_t)SPLIT * HD * ES : 16;
+  static constexpr size_t KS1 = (size_t)SPLIT * KROW * ES, VS1 = (size_t)SPLIT * HD * ES;
   static constexpr size_t KS = SETS * KS1, VS = SETS * VS1, QS = 8 * (size_t)HD * 4, PS = 4 * SETS * SPLIT * 4,
                           WS = 4 * 256 * 4;
   static constexpr size_t BYTES = KS + VS + QS + PS + WS + 16;
@@ -203,12 +203,10 @@ IEK_DEV void kv_load(const __half* p, float* f) {
   }
 }
 
-// One (KV head, head group, chunk) item of the decode attention over an f32 or fp16 cache (T), by
+// head_dim 64 and 128: one (KV head, head group, chunk) item of the decode attention over an f32 or fp16 cache (T), by
 // one 256-thread workgroup: the chunk is `spc` consecutive 64-key slices. Each slice's K and V
 // rows are loaded in one burst of clamped, unconditional 16-byte loads and staged in LDS; the
-// loads of slice i+1 are in flight while slice i is computed. At head dim 512 the K slice fills
-// the LDS, so V goes out once the K rows are staged and is staged in the same buffer after the
-// scores. The GQA group's G query heads split into HG head groups of G / HG (one workgroup each,
+// loads of slice i+1 are in flight while slice i is computed. The GQA group's G query heads split into HG head groups of G / HG (one workgroup each,
 // all streaming the same K / V); wave w takes heads w and w+4 of its group: lane = key for the
 // scores, lane = head dims [DPL*l, DPL*l + DPL) for P.V, with a running (max, sum, o) across the
 // chunk's slices. The chunk publishes its (max, sum, o[]) partials in slot `cp`; the last chunk
@@ -228,10 +226,7 @@ IEK_DEV void attn_chunk(const float* __restrict__ q, const T* __restrict__ kc, c
   constexpr int EPV = 16 / (int)sizeof(T);              // elements per 16-byte load
   constexpr int KROW = AttnSmem<HD, SETS, T>::KROW;     // padded K row: 16-byte reads of different rows spread banks
   constexpr int U4 = SPLIT * HD / EPV;                  // 16-byte loads per K (or V) slice
-  // V is staged in LDS up to head_dim 256; at 512 the K slice, q and V would not fit together, so
-  // the P.V phase reads V rows straight from memory (each row one coalesced 1 KB wave load).
-  constexpr bool VL = HD <= 256;
-  static_assert(HD == 64 || HD == 128 || HD == 256 || HD == 512, "head_dim");
+  static_assert(HD == 64 || HD == 128, "head_dim");
   static_assert(SETS == 1 || SETS == 2, "slice streams");
   const int tid = threadIdx.x & 255, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -240,14 +235,14 @@ IEK_DEV void attn_chunk(const float* __restrict__ q, const T* __restrict__ kc, c
   const int CK = SPLIT * spc;
   const AttnSmem<HD, SETS, T> S(smem);
   auto ks = reinterpret_cast<T(*)[KROW]>(S.ks + (size_t)set * SPLIT * KROW);
-  auto vs = reinterpret_cast<T(*)[VL ? HD : 8]>(S.vs + (VL ? (size_t)set * SPLIT * HD : 0));
+  auto vs = reinterpret_cast<T(*)[HD]>(S.vs + (size_t)set * SPLIT * HD);
   auto qs = reinterpret_cast<float(*)[HD]>(S.qs);
   auto ps = reinterpret_cast<float(*)[SPLIT]>(S.ps + (size_t)set * 4 * SPLIT);
   const T* kh = kc + (size_t)kvh * ctx * HD;
   const T* vh = vc + (size_t)kvh * ctx * HD;
   // native vectors (a HIP uint4 array captured by the lambda would not be promoted to registers)
   typedef uint32_t kv4_t __attribute__((ext_vector_type(4)));
-  kv4_t kr[U4 / 256], vr[VL ? U4 / 256 : 1];
+  kv4_t kr[U4 / 256], vr[U4 / 256];
   // rows [j0, j0 + nk) of the cache; rows past nk repeat row j0 + nk - 1 (nk <= 0: row j0 + nk - 1,
   // within the cache for j0 + nk <= ctx)
   auto issue_rows = [&](int j0, int nk) {
@@ -255,15 +250,7 @@ IEK_DEV void attn_chunk(const float* __restrict__ q, const T* __restrict__ kc, c
     for (int u = 0; u < U4 / 256; ++u) {
       const int i = tid + 256 * u, row = j0 + min(i / (HD / EPV), nk - 1), c8 = i % (HD / EPV);
       kr[u] = *reinterpret_cast<const kv4_t*>(kh + (size_t)row * HD + EPV * c8);
-      if constexpr (VL) vr[u] = *reinterpret_cast<const kv4_t*>(vh + (size_t)row * HD + EPV * c8);
-    }
-  };
-  // head dim 512: the V rows of a slice into the K registers (after the K rows are staged)
-  auto issue_v_rows = [&](int j0, int nk) {
-#pragma unroll
-    for (int u = 0; u < U4 / 256; ++u) {
-      const int i = tid + 256 * u, row = j0 + min(i / (HD / EPV), nk - 1), c8 = i % (HD / EPV);
-      kr[u] = *reinterpret_cast<const kv4_t*>(vh + (size_t)row * HD + EPV * c8);
+      vr[u] = *reinterpret_cast<const kv4_t*>(vh + (size_t)row * HD + EPV * c8);
     }
   };
   // EARLY (no window): the chunk's first slice does not depend on the position, so its rows (all
@@ -305,68 +292,9 @@ IEK_DEV void attn_chunk(const float* __restrict__ q, const T* __restrict__ kc, c
     for (int u = 0; u < U4 / 256; ++u) {
       const int i = tid + 256 * u, row = i / (HD / EPV), c8 = i % (HD / EPV);
       *reinterpret_cast<kv4_t*>(&ks[row][EPV * c8]) = kr[u];
-      if constexpr (VL) *reinterpret_cast<kv4_t*>(&vs[row][EPV * c8]) = vr[u];
+      *reinterpret_cast<kv4_t*>(&vs[row][EPV * c8]) = vr[u];
     }
     __syncthreads();
-    if constexpr (!VL) {
-      // head dim 512: this slice's V rows go out while the scores run, then replace K in LDS
-      issue_v_rows(j0, nk);
-      const bool valid = lane < nk;
-      float pv[2] = {0.f, 0.f}, cv[2] = {1.f, 1.f};
-#pragma unroll
-      for (int t = 0; t < 2; ++t) {
-        const int g = wave + 4 * t;
-        if (g >= GH) break;
-        float sc = 0.f;
-#pragma unroll 8
-        for (int c = 0; c < HD / 8; ++c) {
-          float k8[8];
-          kv_load<8>(&ks[lane][8 * c], k8);
-          const float4 qa = *reinterpret_cast<const float4*>(&qs[g][8 * c]);
-          const float4 qb = *reinterpret_cast<const float4*>(&qs[g][8 * c + 4]);
-          sc += qa.x * k8[0] + qa.y * k8[1] + qa.z * k8[2] + qa.w * k8[3] + qb.x * k8[4] + qb.y * k8[5] +
-                qb.z * k8[6] + qb.w * k8[7];
-        }
-        const float s = valid ? sc * scale : -INFINITY;
-        const float m_new = fmaxf(m_run[t], wave_max(s));
-        cv[t] = m_run[t] == -INFINITY ? 1.f : expf(m_run[t] - m_new);
-        pv[t] = valid ? expf(s - m_new) : 0.f;
-        l_run[t] = l_run[t] * cv[t] + wave_sum(pv[t]);
-        m_run[t] = m_new;
-      }
-      __syncthreads();  // every wave's K reads are done
-#pragma unroll
-      for (int u = 0; u < U4 / 256; ++u) {
-        const int i = tid + 256 * u, row = i / (HD / EPV), c8 = i % (HD / EPV);
-        *reinterpret_cast<kv4_t*>(&ks[row][EPV * c8]) = kr[u];
-      }
-      __syncthreads();
-      if (sb + SETS < sb1) issue(sb + SETS);
-#pragma unroll
-      for (int t = 0; t < 2; ++t) {
-        const int g = wave + 4 * t;
-        if (g >= GH) break;
-        ps[wave][lane] = pv[t];
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        float o[DPL];
-#pragma unroll
-        for (int d = 0; d < DPL; ++d) o[d] = o_run[t][d] * cv[t];
-#pragma unroll 8
-        for (int j = 0; j < nk; ++j) {
-          const float pj = ps[wave][j];
-          float vv[DPL];
-          kv_load<DPL>(&ks[j][DPL * lane], vv);
-#pragma unroll
-          for (int d = 0; d < DPL; ++d) o[d] += pj * vv[d];
-        }
-#pragma unroll
-        for (int d = 0; d < DPL; ++d) o_run[t][d] = o[d];
-        __builtin_amdgcn_wave_barrier();  // ps[wave] is rewritten by the next head
-      }
-      continue;
-    }
     if (sb + SETS < sb1) issue(sb + SETS);
     if (SETS > 1 && sb >= sb1) continue;
     const bool valid = lane < nk;
@@ -479,6 +407,239 @@ IEK_DEV void attn_chunk(const float* __restrict__ q, const T* __restrict__ kc, c
   // stream 1's waves pass a wave index past the group: they take part in the arrival only
   merge_if_last<HD, COH, (SETS > 1)>(part, out, counters, kvh, G, nslot, jmin / CK, (total + CK - 1) / CK,
                                       set ? 8 : wave, S.last, S.wsl, gb, GH, kvh * HG + hg);
+}
+
+// Four consecutive cache elements as raw bits (16 bytes of f32, 8 of fp16) and as floats.
+template <typename T>
+struct Kv4;
+template <>
+struct Kv4<float> {
+  typedef uint32_t raw_t __attribute__((ext_vector_type(4)));
+  IEK_DEV static void get(raw_t r, float (&f)[4]) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) f[i] = __uint_as_float(r[i]);
+  }
+};
+template <>
+struct Kv4<__half> {
+  typedef uint32_t raw_t __attribute__((ext_vector_type(2)));
+  IEK_DEV static void get(raw_t r, float (&f)[4]) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) f[i] = half_bits_to_float(r[i >> 1] >> (16 * (i & 1)));
+  }
+};
+
+// exp(x) for x <= 0 (or -inf, NaN) through the hardware exp2, with the rounding of x * log2(e) put
+// back as a first-order factor (the bare product would cost |x| * 6e-8 of relative error).
+IEK_DEV float exp_neg(float x) {
+  x = x < -256.f ? -256.f : x;  // exp2 is 0 there, and every step below is finite
+  const float L = 1.44269502162933349609375f, L1 = 1.92596299112661746887e-8f;  // log2(e) = L + L1
+  const float t = x * L;
+  const float e = fmaf(x, L1, fmaf(x, L, -t));
+  const float r = __builtin_amdgcn_exp2f(t);
+  return fmaf(r * 0.693147180559945f, e, r);
+}
+
+// Wave sums of four values: row r (lanes 16 r .. 16 r + 15) gets the sum of v_r. Each swap folds
+// two values at once, so this costs ten instructions where four separate sums cost thirty.
+IEK_DEV float wave_sum4(float v0, float v1, float v2, float v3) {
+  auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v0), __float_as_uint(v2), false, false);
+  const float a = __uint_as_float(r[0]) + __uint_as_float(r[1]);  // rows 0, 1: v0; rows 2, 3: v2
+  r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v1), __float_as_uint(v3), false, false);
+  const float b = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+  r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  return row16_sum(__uint_as_float(r[0]) + __uint_as_float(r[1]));
+}
+
+// head_dim 256 and 512: a key's row lies over the wave's 64 lanes, four elements (DV = 2: twice
+// four) each; a wave step is KI keys. A head group is up to four query heads.
+template <int HD>
+struct AttnWide {
+  static constexpr int DV = HD / 256, KI = 4 / DV;
+  static constexpr int UNIT = 4 * KI;  // keys of one step of the workgroup's four waves
+  float o[4][4][HD];
+  float m[4][4], l[4][4];
+  float wsl[4 * 256];
+  int last;
+};
+
+// One (KV head, head group, chunk) item of the decode attention at head_dim 256 and 512 over an f32
+// or fp16 cache (T), by one workgroup of four waves: the chunk is the CK keys from cp * CK, a
+// quarter of them per wave. These are the few-KV-head models, where a step has little to read and
+// latency is the bound: K and V rows go straight to registers in memory order (a wave load is a
+// whole row), the next step's while this one is computed; no LDS and no barrier until the four
+// waves' (max, sum, o) are folded together; chunks down to one step. A group's scores sit one head
+// per 16-lane row, so one exponential serves four heads.
+// The GQA group's G query heads split into head groups of four (one workgroup each). The chunk
+// publishes its (max, sum, o[]) partials in slot `cp`; the last chunk of the (KV head, head group)
+// to finish merges the group's heads (counter kvh * HG + hg). pos_dev: the position (keys - 1) in
+// device memory, else total_in keys; chunks past the live range return at once (uniformly). A chunk
+// that is its KV head's only one (nslot = 1) writes the output itself.
+template <int HD, bool EARLY, typename T>
+IEK_DEV void attn_chunk_wide(const float* __restrict__ q, const T* __restrict__ kc, const T* __restrict__ vc,
+                             float* __restrict__ part, float* __restrict__ out, int* __restrict__ counters, int n_heads,
+                             int n_kv, int ctx, const int* pos_dev, int total_in, int window, float scale, int nslot,
+                             int kvh, int cp, int CK, AttnWide<HD>& S, int hg, int HG) {
+  constexpr int DV = AttnWide<HD>::DV, KI = AttnWide<HD>::KI;
+  typedef typename Kv4<T>::raw_t raw_t;
+  const int tid = threadIdx.x, lane = tid & 63, dl = 4 * lane;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int G = n_heads / n_kv, gb = 4 * hg, GH = min(4, G - gb);
+  const T* kh = kc + (size_t)kvh * ctx * HD + dl;
+  const T* vh = vc + (size_t)kvh * ctx * HD + dl;
+  const int wn = CK / 4, w0 = cp * CK + wave * wn;  // this wave's keys
+  struct Step {
+    raw_t k[KI][DV], v[KI][DV];
+  };
+  // keys kb .. kb + KI - 1, clamped to lo .. hi
+  auto issue = [&](int kb, int lo, int hi, Step& x) {
+#pragma unroll
+    for (int i = 0; i < KI; ++i) {
+      const size_t row = (size_t)max(min(kb + i, hi), lo) * HD;
+#pragma unroll
+      for (int d = 0; d < DV; ++d) {
+        x.k[i][d] = *reinterpret_cast<const raw_t*>(kh + row + 256 * d);
+        x.v[i][d] = *reinterpret_cast<const raw_t*>(vh + row + 256 * d);
+      }
+    }
+  };
+  float qv[4][DV][4];  // (heads past the group's repeat its last one)
+#pragma unroll
+  for (int g = 0; g < 4; ++g)
+#pragma unroll
+    for (int d = 0; d < DV; ++d) {
+      const float4 a =
+          *reinterpret_cast<const float4*>(q + (size_t)(kvh * G + gb + min(g, GH - 1)) * HD + dl + 256 * d);
+      qv[g][d][0] = a.x, qv[g][d][1] = a.y, qv[g][d][2] = a.z, qv[g][d][3] = a.w;
+    }
+  // EARLY (no window): the first step does not depend on the position, so its rows (clamped to the
+  // cache) go out before the position load returns; keys past the live ones are masked below
+  Step st[2];
+  if constexpr (EARLY) issue(w0, 0, ctx - 1, st[0]);
+  typedef __attribute__((address_space(4))) const int* ConstInt;  // a scalar load
+  const int total = pos_dev ? *(ConstInt)pos_dev + 1 : total_in;
+  const int jmin = (window > 0 && total > window) ? total - window : 0;
+  const int c0 = max(cp * CK, jmin), c1 = min(total, (cp + 1) * CK);
+  if (c1 <= c0) return;  // uniform across the workgroup
+  float m = -INFINITY, l = 0.f, o[4][DV][4];  // m, l: head lane / 16
+#pragma unroll
+  for (int g = 0; g < 4; ++g)
+#pragma unroll
+    for (int d = 0; d < DV; ++d)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o[g][d][e] = 0.f;
+  auto of_head = [](float v, int g) {
+    return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v), 16 * g));
+  };
+  auto step = [&](int kb, const Step& x) {
+    float s[KI];
+#pragma unroll
+    for (int i = 0; i < KI; ++i) {
+      float a[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int d = 0; d < DV; ++d) {
+        float kf[4];
+        Kv4<T>::get(x.k[i][d], kf);
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) a[g] = fmaf(qv[g][d][e], kf[e], a[g]);
+      }
+      s[i] = wave_sum4(a[0], a[1], a[2], a[3]);
+      s[i] = kb + i >= c0 && kb + i < c1 ? s[i] * scale : -INFINITY;
+    }
+    float mx = m;
+#pragma unroll
+    for (int i = 0; i < KI; ++i) mx = fmaxf(mx, s[i]);
+    const float base = mx == -INFINITY ? 0.f : mx;  // no finite score yet: every weight is exp(-inf)
+    const float c = exp_neg(m - base);
+    m = mx;
+    l *= c;
+#pragma unroll
+    for (int i = 0; i < KI; ++i) {
+      s[i] = exp_neg(s[i] - base);
+      l += s[i];
+    }
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const float cg = of_head(c, g);
+#pragma unroll
+      for (int d = 0; d < DV; ++d)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[g][d][e] *= cg;
+    }
+#pragma unroll
+    for (int i = 0; i < KI; ++i) {
+      // rows past the live keys may hold anything (0 * inf is NaN): they are left out
+      if (kb + i < c0 || kb + i >= c1) continue;  // uniform
+#pragma unroll
+      for (int d = 0; d < DV; ++d) {
+        float vf[4];
+        Kv4<T>::get(x.v[i][d], vf);
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          const float p = of_head(s[i], g);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) o[g][d][e] = fmaf(p, vf[e], o[g][d][e]);
+        }
+      }
+    }
+  };
+  // the wave's steps that hold live keys
+  const int k_lo = EARLY ? w0 : w0 + max(0, c0 - w0) / KI * KI, k_hi = min(w0 + wn, c1);
+  if (k_lo < k_hi) {
+    if constexpr (!EARLY) issue(k_lo, c0, c1 - 1, st[0]);
+    for (int kb = k_lo; kb < k_hi; kb += 2 * KI) {
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        const int k1 = kb + t * KI;
+        if (k1 >= k_hi) break;
+        if (k1 + KI < k_hi) issue(k1 + KI, c0, c1 - 1, st[t ^ 1]);
+        __builtin_amdgcn_sched_barrier(0);
+        step(k1, st[t]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+  }
+  // fold the four waves' (max, sum, o) through LDS, a thread per (head, dim)
+  if (lane % 16 == 0) {
+    S.m[wave][lane / 16] = m;
+    S.l[wave][lane / 16] = l;
+  }
+#pragma unroll
+  for (int g = 0; g < 4; ++g)
+#pragma unroll
+    for (int d = 0; d < DV; ++d)
+      *reinterpret_cast<float4*>(&S.o[wave][g][dl + 256 * d]) =
+          make_float4(o[g][d][0], o[g][d][1], o[g][d][2], o[g][d][3]);
+  __syncthreads();
+  for (int e = tid; e < GH * HD; e += 256) {
+    const int g = e / HD, d = e % HD;
+    float M = -INFINITY;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) M = fmaxf(M, S.m[t][g]);
+    float L = 0.f, acc = 0.f;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const float mt = S.m[t][g];
+      const float w = mt == -INFINITY ? 0.f : exp_neg(mt - M);  // (a wave without a live key)
+      L += S.l[t][g] * w;
+      acc += S.o[t][g][d] * w;
+    }
+    if (nslot == 1) {
+      out[(size_t)(kvh * G + gb + g) * HD + d] = acc / L;
+    } else {
+      float* pr = part + ((size_t)(kvh * G + gb + g) * nslot + cp) * (HD + 2);
+      if (d == 0) {
+        pr[0] = M;
+        pr[1] = L;
+      }
+      pr[2 + d] = acc;
+    }
+  }
+  if (nslot == 1) return;
+  merge_if_last<HD, false, true>(part, out, counters, kvh, G, nslot, jmin / CK, (total + CK - 1) / CK, wave, &S.last, S.wsl, gb, GH,
+                    kvh * HG + hg);
 }
 
 // Slices per chunk for a cache of `max_len` keys: one up to `target` slices per KV head, then

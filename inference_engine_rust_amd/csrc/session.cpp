@@ -123,8 +123,7 @@ Session::Session(Model* m) : m_(m) {
   actd_ = dev_alloc<float>(fmax);
   tmpd_ = dev_alloc<float>(std::max(qmax, fmax));
   logits_ = dev_alloc<float>(c.vocab);
-  const int nsplit = (ctx_ + 63) / 64;
-  part_ = dev_alloc<float>((size_t)c.n_heads * nsplit * (hdmax + 2));
+  part_ = dev_alloc<float>(attn_decode_part_floats(c.n_heads, hdmax, ctx_));
   d_pos_ = dev_alloc<int>(1);
   d_step_ = dev_alloc<int>(1);
   d_flags_ = dev_alloc<int>(ctx_ + 1);

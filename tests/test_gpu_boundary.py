@@ -173,6 +173,19 @@ def test_dev_attention_decode_matches_oracle(gpu, kv_f32, n_heads, n_kv, hd, tot
         assert rel_l2(got, want) < 2e-6
 
 
+@pytest.mark.parametrize("kv_f32", [False, True])
+@pytest.mark.parametrize("n_heads,n_kv,hd,total,window", [
+    (8, 1, 256, 1, 0), (4, 4, 256, 15, 0), (6, 2, 256, 16, 0), (5, 1, 256, 17, 0), (8, 1, 256, 33, 0),
+    (14, 2, 256, 700, 50), (8, 1, 256, 65, 17), (8, 1, 256, 513, 512), (8, 1, 512, 7, 0), (2, 2, 512, 8, 0),
+    (8, 1, 512, 9, 0), (3, 1, 512, 33, 0), (8, 1, 512, 200, 41), (7, 1, 512, 1030, 0)])
+def test_dev_attention_decode_wide_heads(gpu, kv_f32, n_heads, n_kv, hd, total, window):
+    """head_dim 256 and 512 around the edges of a wave's step, its quarter of a chunk and the chunks,
+    with head groups that fill their four rows and that do not, and live ranges that start inside a
+    step. Bound as for the other decode attention tests: score errors of a few f32 roundings of
+    terms up to ~4, i.e. under 2e-6 relative in the weights."""
+    test_dev_attention_decode_matches_oracle(gpu, kv_f32, n_heads, n_kv, hd, total, window)
+
+
 def test_attention_decode_errors(gpu):
     q, k, v = _att_inputs(8, 2, 64, 4, 0)
     for args, kind in [((8, 2, 64, 0, 0), "Op"), ((8, 3, 64, 4, 0), "Op"), ((8, 2, 96, 4, 0), "Op"),

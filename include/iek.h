@@ -258,8 +258,9 @@ iek_status iek_dev_sample_temperature(const float* logits, size_t n, float tempe
                                       void* stream);
 /* iek_attention_decode over the session's cache layout: k_cache / v_cache are
  * [n_kv_heads][max_seq_len][head_dim] of kv_dtype (IEK_F16 or IEK_F32) with positions
- * [0, total_pos) filled; total_pos <= max_seq_len (IEK_ERR_KV_CACHE otherwise). The partial
- * buffers are allocated per call; waits for the stream before returning. */
+ * [0, total_pos) filled; total_pos <= max_seq_len (IEK_ERR_KV_CACHE otherwise). Waits
+ * for the stream before returning; its scratch is the call's own and kept for later calls (up to
+ * 64 MiB per device, given back by iek_model_free). */
 iek_status iek_dev_attention_decode(const float* q, const void* k_cache, const void* v_cache, int kv_dtype,
                                     size_t n_heads, size_t n_kv_heads, size_t head_dim, size_t max_seq_len,
                                     size_t total_pos, size_t sliding_window, float scale, float* out, void* stream);
@@ -269,15 +270,14 @@ iek_status iek_dev_attention_decode(const float* q, const void* k_cache, const v
  * out[p][h] = softmax(scale * q[p][h] . k[j]) . v[j] over j in [j_min, p], j_min = p -
  * (sliding_window - 1) when 0 < sliding_window, else 0. Runs the session's prefill kernels (fp16
  * (hi, lo) operand pairs on the matrix cores; an input beyond the pairs' range reruns on f32).
- * Supported: head_dim 64, 128, 256 or 512 (IEK_ERR_OP otherwise); seq == 0 is IEK_ERR_OP. Allocates
- * its scratch per call; waits for the stream before returning. */
+ * Supported: head_dim 64, 128, 256 or 512 (IEK_ERR_OP otherwise); seq == 0 is IEK_ERR_OP. Waits
+ * for the stream before returning; scratch as iek_dev_attention_decode. */
 iek_status iek_dev_attention_prefill(const float* q, const float* k, const float* v, size_t seq, size_t n_heads,
                                      size_t n_kv_heads, size_t head_dim, size_t sliding_window, float scale, float* out,
                                      void* stream);
 /* No counterpart in the reference. For callers that cannot allocate device memory (code under
  * HIP graph capture, tight serving loops, harnesses that forbid hipMalloc): iek_dev_attention_decode
- * with the same arguments, results and errors, but its partials, arrival counters and position live
- * in a 16 MiB scratch array the library holds per device until the process ends; it calls no
+ * with the same arguments, results and errors, but its partials and arrival counters live in a 16 MiB scratch array the library holds per device until the process ends; it calls no
  * allocator and does not wait for the stream. Limit: n_heads * ceil(max_seq_len / 64) *
  * (head_dim + 2) * 4 bytes <= 16 MiB - 4 KiB (e.g. 32 heads of 128 up to 32K keys), IEK_ERR_OP
  * beyond. Every call on a device shares that device's scratch: calls that overlap on one GPU (two

@@ -48,6 +48,124 @@ static hipStream_t as_stream(void* s) { return static_cast<hipStream_t>(s); }
 
 static void after_launch() { IEK_HIP(hipGetLastError()); }
 
+// Scratch of the device entries that wait for their stream before they return: a device block and
+// one word of pinned host memory that kernels may store to. A call has its block to itself, and a
+// block is put by for the next call only once the call has waited for its stream (`waited`), so
+// calls of several threads and streams never share one; otherwise it is freed, which waits for the
+// device. With hipMalloc and hipFree in every call a decode attention of 531 keys took 25.4 us (now
+// 22.8), a prefill attention of 2045 x 32 heads of 128 203 (160), of 800 x 8 heads of 256 80 (68). Kept blocks are bounded per device in bytes and number (the oldest go),
+// and all are given back when a model is freed or an allocation here fails.
+// The block starts with SCRATCH_COUNTERS bytes of arrival counters: zero, and left zero by kernels.
+class Scratch {
+ public:
+  static constexpr size_t COUNTERS = 2 * 4096 * 4;  // two per KV head, at most 4096 heads
+  Scratch(size_t bytes, hipStream_t st) {
+    IEK_HIP(hipGetDevice(&b_.device));
+    const size_t need = COUNTERS + bytes;
+    {
+      std::lock_guard<std::mutex> lk(mu());
+      auto& k = kept();
+      auto best = k.end();
+      for (auto i = k.begin(); i != k.end(); ++i)
+        if (i->device == b_.device && i->cap >= need && (best == k.end() || i->cap < best->cap)) best = i;
+      if (best != k.end()) {
+        b_ = *best;
+        k.erase(best);
+        return;
+      }
+    }
+    // rounded up by up to a quarter, so that a length that grows call by call keeps its block
+    size_t step = 64 << 10;
+    while (step * 8 <= need) step *= 2;
+    b_.cap = (need + step - 1) / step * step;
+    if (hipMalloc(&b_.dev, b_.cap) != hipSuccess) {
+      (void)hipGetLastError();
+      b_.dev = nullptr;
+      give_back();
+      IEK_HIP(hipMalloc(&b_.dev, b_.cap));
+    }
+    try {
+      IEK_HIP(hipHostMalloc(reinterpret_cast<void**>(&b_.host), 64, hipHostMallocDefault));
+      launch_fill_i32(reinterpret_cast<int*>(b_.dev), 0, COUNTERS / 4, st);
+      after_launch();
+    } catch (...) {
+      release(b_);
+      throw;
+    }
+  }
+  Scratch(const Scratch&) = delete;
+  Scratch& operator=(const Scratch&) = delete;
+  ~Scratch() {
+    if (!waited_) {
+      release(b_);
+      return;
+    }
+    std::vector<Block> drop;
+    bool held = false;
+    try {
+      std::lock_guard<std::mutex> lk(mu());
+      auto& k = kept();
+      k.push_back(b_);
+      held = true;
+      size_t bytes = 0, n = 0;
+      for (auto& x : k)
+        if (x.device == b_.device) bytes += x.cap, ++n;
+      drop.reserve(n);
+      for (auto i = k.begin(); i != k.end() && (bytes > KEEP_BYTES || n > KEEP_BLOCKS);) {
+        if (i->device != b_.device) {
+          ++i;
+          continue;
+        }
+        bytes -= i->cap, --n;
+        drop.push_back(*i);
+        i = k.erase(i);
+      }
+    } catch (const std::bad_alloc&) {  // not kept, or kept beyond the bound until the next call
+      if (!held) drop.clear(), release(b_);
+    }
+    for (auto& x : drop) release(x);
+  }
+  // The call's work on the block is done.
+  void waited() { waited_ = true; }
+  template <class T>
+  T* at(size_t byte_off = 0) const {
+    return reinterpret_cast<T*>(b_.dev + COUNTERS + byte_off);
+  }
+  int* counters() const { return reinterpret_cast<int*>(b_.dev); }
+  volatile int* host() const { return b_.host; }
+  static void give_back() {
+    std::vector<Block> all;
+    {
+      std::lock_guard<std::mutex> lk(mu());
+      all.swap(kept());
+    }
+    for (auto& x : all) release(x);
+  }
+
+ private:
+  struct Block {
+    char* dev = nullptr;
+    int* host = nullptr;
+    size_t cap = 0;
+    int device = 0;
+  };
+  static constexpr size_t KEEP_BYTES = 64u << 20, KEEP_BLOCKS = 8;
+  static std::mutex& mu() {
+    static std::mutex* m = new std::mutex;  // (never destroyed: calls may outlast static destructors)
+    return *m;
+  }
+  static std::vector<Block>& kept() {
+    static auto* v = new std::vector<Block>;
+    return *v;
+  }
+  static void release(const Block& x) {
+    if (x.dev) (void)hipFree(x.dev);
+    if (x.host) (void)hipHostFree(x.host);
+  }
+  Block b_;
+  bool waited_ = false;
+};
+
 static size_t block_elems(int dt) { return dt == DT_Q8_0 ? 32 : 256; }
 static size_t block_bytes(int dt) { return dt == DT_Q4K ? 144 : dt == DT_Q6K ? 210 : 34; }
 
@@ -69,7 +187,10 @@ iek_status iek_model_load(const char* path, int device, iek_model** out) {
   })
 }
 
-void iek_model_free(iek_model* m) { delete m; }
+void iek_model_free(iek_model* m) {
+  delete m;
+  Scratch::give_back();
+}
 
 iek_status iek_model_load_timings(const iek_model* m, iek_load_timings* o) {
   IEK_API_TRY({
@@ -318,13 +439,13 @@ static size_t attention_check(size_t n_heads, size_t n_kv, size_t hd, size_t max
   return attn_decode_part_floats((int)n_heads, (int)hd, (int)max_len);
 }
 
-// counters (2 * n_kv ints) cleared by a small kernel, so the sequence is safe under stream capture;
-// the length goes by value, and the chunks are sized for it and not for the cache's capacity.
+// clear: the counters (2 * n_kv ints) are cleared by a small kernel first, so the sequence is safe
+// under stream capture (the kernel leaves them zero again); the length goes by value, and the chunks are sized for it and not for the cache's capacity.
 static void attention_launch(const float* q, const void* kc, const void* vc, bool kv_f32, size_t n_heads, size_t n_kv,
                              size_t hd, size_t max_len, size_t total, size_t window, float scale, float* out,
-                             float* part, int* cnt, hipStream_t st) {
+                             float* part, int* cnt, bool clear, hipStream_t st) {
   const int win = window >= total ? 0 : (int)window;  // a window covering every key is no window
-  launch_fill_i32(cnt, 0, 2 * (int)n_kv, st);
+  if (clear) launch_fill_i32(cnt, 0, 2 * (int)n_kv, st);
   launch_attn_decode(q, kc, vc, kv_f32, out, part, cnt, (int)n_heads, (int)n_kv, (int)hd, (int)max_len, nullptr, win,
                      scale, (int)total, st, (int)total);
   after_launch();
@@ -355,19 +476,14 @@ iek_status iek_dev_rope(float* vec, size_t n_heads, uint32_t head_dim, uint32_t 
                         const float* ff, size_t ff_len, void* stream) {
   IEK_API_TRY({
     std::vector<float> cs = rope_table(head_dim, rotary_dim, base, pos, ff, ff_len);
-    float* d = nullptr;
     hipStream_t st = as_stream(stream);
-    IEK_HIP(hipMalloc(&d, std::max<size_t>(cs.size() * 4, 4)));
-    try {
-      IEK_HIP(hipMemcpyAsync(d, cs.data(), cs.size() * 4, hipMemcpyHostToDevice, st));
-      launch_rope_rows(vec, 1, (int)(n_heads * head_dim), (int)n_heads, (int)head_dim, 0, d, (int)(cs.size() / 2), st);
-      after_launch();
-      IEK_HIP(hipStreamSynchronize(st));
-    } catch (...) {
-      (void)hipFree(d);
-      throw;
-    }
-    IEK_HIP(hipFree(d));
+    Scratch s(cs.size() * 4, st);
+    float* d = s.at<float>();
+    IEK_HIP(hipMemcpyAsync(d, cs.data(), cs.size() * 4, hipMemcpyHostToDevice, st));
+    launch_rope_rows(vec, 1, (int)(n_heads * head_dim), (int)n_heads, (int)head_dim, 0, d, (int)(cs.size() / 2), st);
+    after_launch();
+    IEK_HIP(hipStreamSynchronize(st));
+    s.waited();
   })
 }
 
@@ -403,15 +519,9 @@ iek_status iek_dev_residual_add(const float* a, const float* b, float* out, size
 iek_status iek_dev_argmax(const float* logits, size_t n, uint32_t* out_index, void* stream) {
   IEK_API_TRY({
     if (n == 0) fail(ST_SAMPLING, "logits slice is empty");
-    unsigned long long* key = nullptr;
-    IEK_HIP(hipMalloc(&key, 64));
-    try {
-      *out_index = argmax_dev(logits, n, key, as_stream(stream));
-    } catch (...) {
-      (void)hipFree(key);
-      throw;
-    }
-    IEK_HIP(hipFree(key));
+    Scratch s(64, as_stream(stream));
+    *out_index = argmax_dev(logits, n, s.at<unsigned long long>(), as_stream(stream));
+    s.waited();
   })
 }
 
@@ -430,15 +540,9 @@ iek_status iek_dev_sample_temperature(const float* logits, size_t n, float tempe
                                       void* stream) {
   IEK_API_TRY({
     if (n == 0) fail(ST_SAMPLING, "logits slice is empty");
-    uint32_t* word = nullptr;
-    IEK_HIP(hipMalloc(&word, 64));
-    try {
-      *out_index = sample_dev(logits, n, temperature, r, word, as_stream(stream));
-    } catch (...) {
-      (void)hipFree(word);
-      throw;
-    }
-    IEK_HIP(hipFree(word));
+    Scratch s(64, as_stream(stream));
+    *out_index = sample_dev(logits, n, temperature, r, s.at<uint32_t>(), as_stream(stream));
+    s.waited();
   })
 }
 
@@ -450,19 +554,11 @@ iek_status iek_dev_attention_decode(const float* q, const void* k_cache, const v
     attention_check(n_heads, n_kv_heads, head_dim, max_seq_len, total_pos);
     const size_t pf = attn_decode_part_floats((int)n_heads, (int)head_dim, (int)total_pos);
     hipStream_t st = as_stream(stream);
-    char* scratch = nullptr;
-    const size_t cnt_off = (pf * 4 + 255) / 256 * 256;
-    IEK_HIP(hipMalloc(&scratch, cnt_off + 2 * n_kv_heads * 4));
-    try {
-      int* cnt = reinterpret_cast<int*>(scratch + cnt_off);
-      attention_launch(q, k_cache, v_cache, kv_dtype == IEK_F32, n_heads, n_kv_heads, head_dim, max_seq_len, total_pos,
-                       sliding_window, scale, out, reinterpret_cast<float*>(scratch), cnt, st);
-      IEK_HIP(hipStreamSynchronize(st));  // the scratch is freed below
-    } catch (...) {
-      (void)hipFree(scratch);
-      throw;
-    }
-    IEK_HIP(hipFree(scratch));
+    Scratch s(pf * 4, st);
+    attention_launch(q, k_cache, v_cache, kv_dtype == IEK_F32, n_heads, n_kv_heads, head_dim, max_seq_len, total_pos,
+                     sliding_window, scale, out, s.at<float>(), s.counters(), false, st);
+    IEK_HIP(hipStreamSynchronize(st));
+    s.waited();
   })
 }
 
@@ -479,28 +575,20 @@ iek_status iek_dev_attention_prefill(const float* q, const float* k, const float
     const int M = (int)seq, nh = (int)n_heads, nkv = (int)n_kv_heads, hd = (int)head_dim;
     const int win = sliding_window >= seq ? 0 : (int)sliding_window;  // a window covering every key is no window
     hipStream_t st = as_stream(stream);
-    // the K / V^T fp16 planes of the shared-K/V kernel (head_dim up to 256), then the range flag
+    // the K / V^T fp16 planes of the shared-K/V kernel (head_dim up to 256); kernels only ever store
+    // to the range flag, so it is the scratch's host word (no clearing launch, no copy back)
     const size_t halves = hd <= 256 ? attn_prefill_scratch_halves(M, nkv, hd) : 0;
-    const size_t ovf_off = (halves * 2 + 255) / 256 * 256;
-    char* scratch = nullptr;
-    IEK_HIP(hipMalloc(&scratch, ovf_off + 256));
-    try {
-      int* ovf = reinterpret_cast<int*>(scratch + ovf_off);
-      launch_fill_i32(ovf, 0, 1, st);
-      launch_attn_prefill(q, k, v, out, M, nh, nkv, hd, win, scale, st, halves ? scratch : nullptr, halves, false, ovf);
-      int flagged = 0;
-      IEK_HIP(hipMemcpyAsync(&flagged, ovf, sizeof(int), hipMemcpyDeviceToHost, st));
+    Scratch s(halves * 2, st);
+    *s.host() = 0;
+    launch_attn_prefill(q, k, v, out, M, nh, nkv, hd, win, scale, st, halves ? s.at<char>() : nullptr, halves, false,
+                        const_cast<int*>(s.host()));
+    IEK_HIP(hipStreamSynchronize(st));
+    // an input beyond the fp16 pair's range: the f32 kernel, as the session's prefill reruns
+    if (*s.host()) {
+      launch_attn_prefill_f32(q, k, v, out, M, nh, nkv, hd, win, scale, st);
       IEK_HIP(hipStreamSynchronize(st));
-      // an input beyond the fp16 pair's range: the f32 kernel, as the session's prefill reruns
-      if (flagged) {
-        launch_attn_prefill_f32(q, k, v, out, M, nh, nkv, hd, win, scale, st);
-        IEK_HIP(hipStreamSynchronize(st));
-      }
-    } catch (...) {
-      (void)hipFree(scratch);
-      throw;
     }
-    IEK_HIP(hipFree(scratch));
+    s.waited();
   })
 }
 
@@ -521,7 +609,7 @@ iek_status iek_dev_attention_decode_noalloc(const float* q, const void* k_cache,
     int* cnt = reinterpret_cast<int*>(base);
     float* part = reinterpret_cast<float*>(base + NOALLOC_COUNTER_BYTES);
     attention_launch(q, k_cache, v_cache, kv_dtype == IEK_F32, n_heads, n_kv_heads, head_dim, max_seq_len, total_pos,
-                     sliding_window, scale, out, part, cnt, as_stream(stream));
+                     sliding_window, scale, out, part, cnt, true, as_stream(stream));
   })
 }
 
@@ -734,7 +822,7 @@ iek_status iek_attention_decode(const float* q, const float* k_cache, const floa
     const float* dv = hc.up<float>(2, vt.data(), kvn * 4);
     int* cnt = hc.ptr<int>(5);
     attention_launch(dq, dk, dv, true, n_heads, n_kv_heads, head_dim, total_pos, total_pos, sliding_window, scale,
-                     hc.ptr<float>(3), hc.ptr<float>(4), cnt, hc.st);
+                     hc.ptr<float>(3), hc.ptr<float>(4), cnt, true, hc.st);
     hc.down(out, hc.ptr<float>(3), qn);
     hc.finish();
   })

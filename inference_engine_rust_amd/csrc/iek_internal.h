@@ -189,7 +189,7 @@ void launch_attn_decode(const float* q, const void* kc, const void* vc, bool kv_
 // Floats of `part` that launch_attn_decode needs at most for a cache of max_len keys.
 size_t attn_decode_part_floats(int n_heads, int head_dim, int max_len);
 // The no-allocation scratch (kernels/noalloc.hip): a file-scope device array of this many bytes
-// per device, [counters + position: NOALLOC_COUNTER_BYTES][attention partials: the rest].
+// per device, [counters: NOALLOC_COUNTER_BYTES][attention partials: the rest].
 constexpr size_t NOALLOC_SCRATCH_BYTES = 16u << 20;
 constexpr size_t NOALLOC_COUNTER_BYTES = 4096;
 // Device address of the scratch array of the stream's device (the current device for the null

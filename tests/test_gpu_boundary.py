@@ -186,6 +186,51 @@ def test_dev_attention_decode_wide_heads(gpu, kv_f32, n_heads, n_kv, hd, total, 
     test_dev_attention_decode_matches_oracle(gpu, kv_f32, n_heads, n_kv, hd, total, window)
 
 
+@pytest.mark.parametrize("totals", [(40, 4000, 41), (3000, 65, 3001, 66, 9000, 67)])
+def test_waiting_entries_share_scratch_between_threads(gpu, totals):
+    """The waiting entries keep their scratch for the next call: sizes that grow and shrink, decode
+    and prefill attention in turn, from three threads with a stream each, give the same bits as one
+    call after another."""
+    import threading
+    n_heads, n_kv, hd = 8, 2, 128
+    rng = np.random.default_rng(5)
+    top = max(totals)
+    q, k, v = (torch.from_numpy(rng.standard_normal((top, h, hd)).astype(np.float32)).to("cuda")
+               for h in (n_heads, n_kv, n_kv))
+    torch.cuda.synchronize()
+
+    def calls(stream):
+        got = []
+        for t in totals:
+            out = torch.zeros(n_heads * hd, dtype=torch.float32, device="cuda")
+            pre = torch.zeros(min(t, 200), n_heads, hd, dtype=torch.float32, device="cuda")
+            torch.cuda.current_stream().synchronize()
+            E.attention_decode(q.data_ptr(), k.data_ptr(), v.data_ptr(), E.F32, n_heads, n_kv, hd, top // n_kv, t // n_kv,
+                               0, 0.09, out.data_ptr(), stream)
+            E.attention_prefill(q.data_ptr(), k.data_ptr(), v.data_ptr(), pre.shape[0], n_heads, n_kv, hd, 0, 0.09,
+                                pre.data_ptr(), stream)
+            got += [out.cpu(), pre.cpu()]
+        return got
+
+    want = calls(torch.cuda.current_stream().cuda_stream)
+    streams = [torch.cuda.Stream() for _ in range(3)]
+    got = [[] for _ in streams]
+
+    def work(i):
+        for _ in range(4):
+            got[i].append(calls(streams[i].cuda_stream))
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(3)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for runs in got:
+        assert len(runs) == 4
+        for r in runs:
+            assert all(torch.equal(a, b) for a, b in zip(r, want))
+
+
 def test_attention_decode_errors(gpu):
     q, k, v = _att_inputs(8, 2, 64, 4, 0)
     for args, kind in [((8, 2, 64, 0, 0), "Op"), ((8, 3, 64, 4, 0), "Op"), ((8, 2, 96, 4, 0), "Op"),

@@ -140,8 +140,8 @@ void launch_range_flag3(const float* a, size_t na, const float* b, const float* 
 // Op-level GEMM inputs with any f32 range: per row, the power-of-two factor s (1 unless the row's
 // largest |value| or per-32 sum exceeds 2^15, then the factor that brings it into [2^14, 2^15)),
 // the fp16 (hi, lo) planes of s * a and the per-32 sums of s * a (fp16 pair planes), and
-// inv[m] = 1 / s. Then launch_row_scale multiplies each output row by inv[m]; power-of-two factors
-// make both steps exact.
+// inv[m] = 1 / s. Then each output row is multiplied by inv[m] (launch_gemm_q's row_scale, or
+// launch_row_scale); power-of-two factors make both steps exact.
 // With `cnt`, `ncnt` ints there are cleared.
 void launch_split_scaled(const float* a, int rows, int K, __half* hi, __half* lo, float* sums, float* inv, int* cnt,
                          int ncnt, hipStream_t st);

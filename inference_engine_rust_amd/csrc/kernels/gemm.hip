@@ -109,11 +109,11 @@ void launch_gemm(int dt, const void* w, const float* a, int M, int K, int N, flo
     }
     GemmQSeg seg{wq, out, N};
     launch_gemm_q(wdt, &seg, 1, xh, xh + n, xs, M, K, nullptr, st, reinterpret_cast<float*>(base + xbytes + ibytes),
-                  false, skinny ? inv : nullptr, sks ? &sk : nullptr);
+                  false, inv, sks ? &sk : nullptr);
   } else {
     launch_gemm_mfma(dt, w, xh, xh + n, M, K, N, out, nullptr, st);
+    launch_row_scale(out, M, N, inv, st);
   }
-  if (!skinny) launch_row_scale(out, M, N, inv, st);
   check_hip(hipFreeAsync(buf, st), "hipFreeAsync");
 }
 

@@ -98,6 +98,12 @@ struct QDeq<DT_Q8_0> {
   }
 };
 
+// The output factors of rows m .. m + 3 (1 without them; rows past M are not written).
+IEK_DEV void row_factors(const float* row_scale, int m, int M, float (&f)[4]) {
+#pragma unroll
+  for (int r = 0; r < 4; ++r) f[r] = row_scale ? row_scale[min(m + r, M - 1)] : 1.f;
+}
+
 template <int DT, int BM, int BN>
 __global__ __launch_bounds__(256) void gemm_q_kernel(GemmQArgs g) {
   constexpr int WM = BM / 4, MT = WM / 16, NT = BN / 16;
@@ -256,7 +262,9 @@ __global__ __launch_bounds__(256) void gemm_q_kernel(GemmQArgs g) {
 
   const float* resid = s == 0 ? g.resid : nullptr;
 #pragma unroll
-  for (int i = 0; i < MT; ++i)
+  for (int i = 0; i < MT; ++i) {
+    float f[4];
+    row_factors(g.row_scale, m0 + wave * WM + 16 * i + 4 * (lane >> 4), M, f);
 #pragma unroll
     for (int j = 0; j < NT; ++j) {
       const int n = n0 + 16 * j + fr;
@@ -264,12 +272,13 @@ __global__ __launch_bounds__(256) void gemm_q_kernel(GemmQArgs g) {
       for (int r = 0; r < 4; ++r) {
         const int m = m0 + wave * WM + 16 * i + 4 * (lane >> 4) + r;
         if (m < M && n < N) {
-          float v = acc[i][j][r];
+          float v = acc[i][j][r] * f[r];
           if (resid) v = resid[(size_t)m * N + n] + v;
           out[(size_t)m * N + n] = v;
         }
       }
     }
+  }
 }
 
 // ---- K-quants: 64 x 64 wave tiles, weights dequantised straight into MFMA operand registers ----
@@ -428,6 +437,11 @@ IEK_DEV void kq_deq(int p, int h, const typename T::Hdr& hd, const typename T::R
   }
 }
 
+// Swizzle of an activation row's eight 16-byte chunks in LDS: the rows that eight lanes of an operand
+// read touch get all eight chunk positions, and the two rows whose four chunks eight lanes store (the
+// planes' tile order) get opposite halves.
+IEK_DEV int a_swz(int row) { return ((row & 1) << 2) | ((row >> 1) & 3); }
+
 // TM: 16-row MFMA tiles per wave along M (a wave owns 16 TM x 64); WGM x WGN waves.
 // OCC: waves per SIMD the register allocation must allow (2 caps each wave at 256 registers).
 // FM, how the superblock factor d enters the f32 sum:
@@ -523,7 +537,7 @@ __global__ __launch_bounds__(64 * WGM * WGN, OCC) void gemm_kq_kernel(GemmQArgs 
   auto store_a = [&](int buf, const ASlot& sl) {
 #pragma unroll
     for (int u = 0; u < AR; ++u) {
-      const int ch = as_row[u] * 8 + (as_c[u] ^ (as_row[u] & 7));
+      const int ch = as_row[u] * 8 + (as_c[u] ^ a_swz(as_row[u]));
       As[buf][ch] = sl.a[u];
       As[buf][PL + ch] = sl.a[AR + u];
     }
@@ -589,7 +603,7 @@ __global__ __launch_bounds__(64 * WGM * WGN, OCC) void gemm_kq_kernel(GemmQArgs 
           const int row = WR * wm + 16 * i + lr;
 #pragma unroll
           for (int hh = 0; hh < 2; ++hh) {
-            const int ch = row * 8 + ((4 * hh + lg) ^ (row & 7));
+            const int ch = row * 8 + ((4 * hh + lg) ^ a_swz(row));
             x[2 * hh] = As[buf][ch];
             x[2 * hh + 1] = As[buf][PL + ch];
           }
@@ -651,7 +665,7 @@ __global__ __launch_bounds__(64 * WGM * WGN, OCC) void gemm_kq_kernel(GemmQArgs 
         // activation operands one m-tile ahead of the MFMAs that use them
         qu4_t ah[2], al[2];
         auto rd = [&](int i, qu4_t& x, qu4_t& y) {
-          const int row = WR * wm + 16 * i + lr, ch = row * 8 + ((4 * h + lg) ^ (row & 7));
+          const int row = WR * wm + 16 * i + lr, ch = row * 8 + ((4 * h + lg) ^ a_swz(row));
           x = As[buf][ch];
           y = As[buf][PL + ch];
         };
@@ -732,6 +746,15 @@ __global__ __launch_bounds__(256) void add_part_kernel(float* __restrict__ out, 
   }
 }
 
+// The same with the row factors: out[m] = (out[m] + part[m]) * scale[m].
+__global__ __launch_bounds__(256) void add_part_scale_kernel(float* __restrict__ out, const float* __restrict__ part,
+                                                            const float* __restrict__ scale, int N) {
+  const size_t row = (size_t)blockIdx.y * N;
+  const float f = scale[blockIdx.y];
+  for (int i = blockIdx.x * 256 + threadIdx.x; i < N; i += gridDim.x * 256)
+    out[row + i] = (out[row + i] + part[row + i]) * f;
+}
+
 }  // namespace
 
 bool gemm_q_ok(int dt, const void* w, int K) {
@@ -782,7 +805,14 @@ static bool gemm_kq_launch(GemmQArgs g, hipStream_t st, bool defer_add) {
                      0, st, g);
   if (g.ksplit == 2) {
     if (defer_add) return true;
-    launch_add_f32(g.out[0], g.kpart, mn, st);
+    if (g.row_scale)
+      hipLaunchKernelGGL(add_part_scale_kernel, dim3((unsigned)std::min((g.n[0] + 255) / 256, 64), g.M), dim3(256), 0,
+                         st, g.out[0], g.kpart, g.row_scale, g.n[0]);
+    else
+      launch_add_f32(g.out[0], g.kpart, mn, st);
+  } else if (g.row_scale) {
+    // (in the epilogue the factors' registers cost every other GEMM of this kernel 2 to 5%)
+    for (int i = 0; i < g.nseg; ++i) launch_row_scale(g.out[i], g.M, g.n[i], g.row_scale, st);
   }
   return false;
 }
@@ -855,7 +885,9 @@ void launch_add_f32(float* out, const float* part, size_t n, hipStream_t st) {
 }
 
 bool launch_gemm_q(int dt, const GemmQSeg* segs, int nseg, const __half* xh, const __half* xl, const float* xs, int M,
-                   int K, const float* resid, hipStream_t st, float* kpart, bool defer_add, const float* row_scale, const SkScratch* sk) {
+                   int K, const float* resid, hipStream_t st, float* kpart, bool defer_add, const float* row_scale,
+                   const SkScratch* sk) {
+  if (row_scale && (resid || defer_add)) fail(ST_OP, "gemm_q: row factors apply to the finished sum");
   if (nseg < 1 || nseg > 3 || M < 1) fail(ST_OP, "gemm_q: 1..3 segments and M >= 1");
   GemmQArgs g{};
   g.nseg = nseg;
@@ -872,6 +904,7 @@ bool launch_gemm_q(int dt, const GemmQSeg* segs, int nseg, const __half* xh, con
   g.xs = xs;
   g.resid = resid;
   g.kpart = kpart;
+  g.row_scale = row_scale;
   g.ksplit = 1;
   const size_t nsb = (size_t)(K / QK_K);
   switch (dt) {
@@ -884,7 +917,6 @@ bool launch_gemm_q(int dt, const GemmQSeg* segs, int nseg, const __half* xh, con
   int ncols = 0;
   for (int i = 0; i < nseg; ++i) ncols += segs[i].n;
   if (gemm_skinny_ok(dt, M, ncols)) {
-    g.row_scale = row_scale;
     g.kpart = sk ? sk->part : nullptr;
     g.sk_cnt = sk ? sk->cnt : nullptr;
     launch_gemm_skinny(dt, g, false, st);

@@ -29,13 +29,15 @@ __global__ void repack_q6k_kernel(const uint8_t* __restrict__ src, int nsb, int 
     uint8_t* d = row + (size_t)nsb * 208 + 2 * j;
     d[0] = blk[208];
     d[1] = blk[209];
+    // the row's last superblock zeroes the padding behind the factors
+    if (j == nsb - 1)
+      for (uint8_t* z = d + 2; z < row + q6r_row_bytes(nsb); ++z) *z = 0;
   }
 }
 
 void launch_repack_q6k(const void* src, int K, int N, void* dst, hipStream_t st) {
   if (K % QK_K != 0) fail(ST_OP, "repack_q6k: K must be a multiple of 256");
   const int nsb = K / QK_K;
-  IEK_HIP(hipMemsetAsync(dst, 0, (size_t)N * q6r_row_bytes(nsb), st));
   const size_t threads = (size_t)N * nsb * 4;
   hipLaunchKernelGGL(repack_q6k_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, st,
                      (const uint8_t*)src, nsb, N, (uint8_t*)dst);
@@ -52,12 +54,13 @@ __global__ void repack_q80_kernel(const uint8_t* __restrict__ src, int nb, int N
   for (int t = 0; t < 32; ++t) row[32 * b + t] = blk[2 + t];
   row[(size_t)32 * nb + 2 * b] = blk[0];
   row[(size_t)32 * nb + 2 * b + 1] = blk[1];
+  if (b == nb - 1)
+    for (uint8_t* z = row + (size_t)34 * nb; z < row + q8r_row_bytes(nb); ++z) *z = 0;
 }
 
 void launch_repack_q80(const void* src, int K, int N, void* dst, hipStream_t st) {
   if (K % Q8_0_ELEMS != 0) fail(ST_OP, "repack_q80: K must be a multiple of 32");
   const int nb = K / Q8_0_ELEMS;
-  IEK_HIP(hipMemsetAsync(dst, 0, (size_t)N * q8r_row_bytes(nb), st));
   const size_t threads = (size_t)N * nb;
   hipLaunchKernelGGL(repack_q80_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, st,
                      (const uint8_t*)src, nb, N, (uint8_t*)dst);

@@ -42,6 +42,7 @@ SOURCES = [
     "kernels/gemm_mfma.hip",
     "kernels/gemm_q.hip",
     "kernels/gemm_skinny.hip",
+    "kernels/gemm_q80.hip",
     "kernels/gemma.hip",
     "kernels/chain.hip",
     "kernels/noalloc.hip",

@@ -13,7 +13,10 @@
 // three (+ a_hi*w'_lo). The superblock factor d (Q8_0: per 32) multiplies a per-superblock MFMA
 // accumulator into the output accumulator; Q4_K's min term uses the per-32 row sums of a.
 //
-// Tiling: BM x BN outputs per 256-thread workgroup (64x64 .. 128x128), four waves stacked along M;
+// Q8_0 runs in gemm_q80.hip, few rows of any type in gemm_skinny.hip.
+//
+// Tiling of native Q6_K (tensors without a regrouped copy): BM x BN outputs per 256-thread workgroup,
+// four waves stacked along M;
 // 32-wide K stages double-buffered in LDS (one barrier per stage) with the next stage's raw bytes
 // in flight in registers while the current stage's MFMAs run. Up to three weight matrices that
 // share the activation (Q/K/V) run as one launch; M tiles of one N tile share an XCD's L2.
@@ -73,28 +76,6 @@ struct QDeq<DT_Q6K> {
     }
     hi = make_uint4(hpack(h[0], h[2]), hpack(h[1], h[3]), hpack(h[4], h[6]), hpack(h[5], h[7]));  // plane_pos order
     lo = make_uint4(hpack(l[0], l[2]), hpack(l[1], l[3]), hpack(l[4], l[6]), hpack(l[5], l[7]));
-  }
-};
-
-template <>
-struct QDeq<DT_Q8_0> {
-  static constexpr int PERIOD = 1;
-  static constexpr bool LO = false;
-  uint32_t q[4], d16;
-  IEK_DEV void load(const uint8_t* w, size_t row_bytes, int n, int k0, int nsb) {
-    const uint8_t* blk = w + (size_t)n * row_bytes + (size_t)(k0 >> 5) * Q8_0_BYTES;
-    const uint16_t* p = reinterpret_cast<const uint16_t*>(blk + 2 + (k0 & 31));
-#pragma unroll
-    for (int i = 0; i < 4; ++i) q[i] = p[i];
-    d16 = *reinterpret_cast<const uint16_t*>(blk);
-  }
-  IEK_DEV void decode(int, uint4& hi, uint4& lo, float& d) const {
-    d = half_bits_to_float(d16);
-    _Float16 h[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) h[i] = (_Float16)(int)(int8_t)((q[i >> 1] >> (8 * (i & 1))) & 0xFFu);
-    hi = make_uint4(hpack(h[0], h[2]), hpack(h[1], h[3]), hpack(h[4], h[6]), hpack(h[5], h[7]));  // plane_pos order
-    lo = make_uint4(0, 0, 0, 0);
   }
 };
 
@@ -926,7 +907,7 @@ bool launch_gemm_q(int dt, const GemmQSeg* segs, int nseg, const __half* xh, con
     case DT_Q4K: return gemm_kq<Q4KB>(g, st, defer_add);
     case DT_Q6K: gemm_q_dt<DT_Q6K>(g, st); return false;
     case DT_Q6K_R: return gemm_kq<Q6RB>(g, st, defer_add);
-    default: gemm_q_dt<DT_Q8_0>(g, st); return false;
+    default: launch_gemm_q80(g, st); return false;
   }
 }
 

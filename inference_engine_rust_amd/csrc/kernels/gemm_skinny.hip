@@ -556,14 +556,18 @@ void skinny(GemmQArgs& g, bool glu, hipStream_t st) {
 // 4096 x 4096 at 23 rows 13 / 46, 64 rows 22 / 48, 128 rows 30 / 52; 14336 x 4096 at 23 rows 24 / 48,
 // 64 rows 44 / 46, 128 rows 86 / 57. Q6_K 4096 x 14336 at 23 rows 30 / 220, 64 rows 47 / 221, 128
 // rows 83 / 227 (its tiles take three MFMAs per product and K = 14336 on 32 workgroups). Q8_0
-// 6144 x 1536 at 23 rows 13 / 29, 64 rows 14 / 30, 128 rows 26 / 30; 1536 x 6144 at 13 rows 11 / 92.
+// 6144 x 1536 at 23 rows 13 / 29; 1536 x 6144 at 13 rows 11 / 92. Q8_0 above 32 rows takes two or
+// more passes of 32 here, and gemm_q80.hip's tiles are as fast once they are enough of them (whole
+// op-level calls, this kernel / those): 64 rows 4096 x 14336 65 / 92, 1536 x 6144 34 / 45, 6144 x 1536
+// 31 / 24, 14336 x 4096 62 / 43; 128 rows 512 x 4096 25 / 38, 1536 x 6144 51 / 49, 1536 x 2048
+// 28 / 26, 6144 x 1536 41 / 34, 4096 x 14336 113 / 93.
 bool gemm_skinny_ok(int dt, int M, int N) {
   const long long c = (long long)N * ((M + 63) / 64);
   switch (dt) {
     case DT_Q4K: return M <= 32 || (M <= 128 && c <= 8192);
     case DT_Q6K:
     case DT_Q6K_R: return M <= 64 || (M <= SK_MAX_ROWS && c <= 16384);
-    case DT_Q8_0: return M <= 128;
+    case DT_Q8_0: return M <= 32 || (M <= 128 && (long long)N * ((M + 31) / 32) <= (M <= 64 ? 8192 : 5120));
     default: return false;
   }
 }

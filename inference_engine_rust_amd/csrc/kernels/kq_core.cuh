@@ -162,5 +162,6 @@ IEK_DEV void glu_epilogue(const GemmQArgs& g, const AccT& acc, const float (&Dc)
 }  // namespace
 
 void launch_gemm_skinny(int dt, GemmQArgs& g, bool glu, hipStream_t st);
+void launch_gemm_q80(GemmQArgs& g, hipStream_t st);
 
 }  // namespace iek

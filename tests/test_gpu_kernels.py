@@ -155,6 +155,15 @@ def test_gemm_few_rows(gpu, dt, k, n, m):
     _check_matmul(dt, k, n, m, seed=5)
 
 
+@pytest.mark.parametrize("k,n,m", [
+    # waves without a unit of K, partial units (K % 128) whose last row ends the tensor, ragged columns
+    (32, 40, 129), (96, 65, 190), (160, 1733, 100), (512, 63, 193), (544, 70, 256),
+    # ragged row tiles (a tile of one row, of 16, of 63), whole tiles, both sides of the few-row kernel's range
+    (1408, 130, 129), (288, 128, 144), (1536, 64, 319), (384, 4100, 40), (384, 4096, 64), (256, 1280, 128)])
+def test_gemm_q80_tiles(gpu, k, n, m):
+    _check_matmul(E.Q8_0, k, n, m, seed=8)
+
+
 @pytest.mark.parametrize("dt,k,n,m", [(E.Q4K, 4096, 1024, 7), (E.Q6K, 1024, 130, 24), (E.Q8_0, 1408, 64, 40)])
 def test_gemm_few_rows_full_f32_range(gpu, dt, k, n, m):
     _check_matmul(dt, k, n, m, seed=6, a=_wide_range_rows(m, k, 60 + dt))

@@ -7,6 +7,7 @@
 //
 // Prefill (attention.rs:175-422): causal attention over the f32 K/V of the prompt (the
 // reference attends to the layer's own k_data/v_data, not the cache).
+#include <algorithm>
 #include <cmath>
 #include <type_traits>
 
@@ -88,10 +89,12 @@ static void attn_decode_wide(hipStream_t st, const float* q, const T* kc, const 
   // Keys per chunk: a chunk's time grows with its keys and the merge's with the number of chunks,
   // so about sqrt(2 * keys) of them (a window keeps only ~window keys live). Measured with 16 / 32 /
   // 64 chunks per KV head, one KV head of 512: 11.8 / 13.3 / 17.5 us at 500 keys, 20.2 / 17.3 / 19.9
-  // at 2000, 49 / 33 / 28 at 8000. In whole steps of the workgroup, within the partial slots.
+  // at 2000, 49 / 33 / 28 at 8000. In whole steps of the workgroup, within the partial slots and with at
+  // most MERGE_SLOTS live chunks (a window touches one more than its own length holds).
   constexpr int UNIT = AttnWide<HD>::UNIT;
   const int span = window > 0 ? std::min(max_len, window) : max_len, slots = attn_slots(n_heads, HD, max_len);
-  const int keys = std::max((int)std::sqrt(2.0 * span), (max_len + slots - 1) / slots);
+  const int keys = std::max({(int)std::sqrt(2.0 * span), (max_len + slots - 1) / slots,
+                             (span + MERGE_SLOTS - 2) / (MERGE_SLOTS - 1)});
   const int CK = (keys + UNIT - 1) / UNIT * UNIT, nchunk = (max_len + CK - 1) / CK;
   auto go = [&](auto kern) {
     hipLaunchKernelGGL(kern, dim3(n_kv * HG, nchunk), dim3(256), 0, st, q, kc, vc, part, out, counters, n_heads, n_kv,

@@ -9,6 +9,9 @@
 namespace iek {
 
 constexpr int SPLIT = 64;
+// Live partials of a query head that one merge takes: it stages their weights in LDS. The chunk sizes
+// are chosen (attention.hip) so that no launch leaves more of them.
+constexpr int MERGE_SLOTS = 256;
 
 // One 256-thread workgroup per (KV head, 64-key slice): the four waves load the slice's K and V
 // rows (fp16) into LDS together in one burst of clamped, unconditional 16-byte loads, then wave w
@@ -19,13 +22,13 @@ constexpr int SPLIT = 64;
 // Merge of the live slice partials of query head h by one wave: global (max, sum) over slices,
 // then each lane folds its head dims of every slice with the rescaled weights. One round trip
 // fetches lane s's (max, sum) pair together with the first batch of B o rows; further batches
-// follow only for more than B live slots.
+// follow only for more than B live slots (at most MERGE_SLOTS).
 template <int HD, bool COH = false, int B = (HD >= 512 ? 4 : 2048 / HD)>
 IEK_DEV void merge_head(const float* __restrict__ part, float* __restrict__ out, int h, int nsplit, int s0, int nlive,
                         float* wsl) {
   constexpr int DPL = HD / 64;
   const int lane = threadIdx.x & 63;
-  const int ns = min(nlive - s0, 256);
+  const int ns = nlive - s0;
   const float* pr = part + ((size_t)h * nsplit + s0) * (HD + 2);
   const int sl = min(lane, ns - 1);
   const float m_l = ld_f<COH>(pr + (size_t)sl * (HD + 2));
@@ -73,12 +76,6 @@ IEK_DEV void merge_head(const float* __restrict__ part, float* __restrict__ out,
       }
     }
   }
-  // slices beyond the 256 staged weights (contexts over 16K keys) use direct weights
-  for (int s = 256; s < nlive - s0; ++s) {
-    const float w = expf(ld_f<COH>(pr + (size_t)s * (HD + 2)) - M);
-#pragma unroll
-    for (int t = 0; t < DPL; ++t) acc[t] += ld_f<COH>(pr + (size_t)s * (HD + 2) + 2 + DPL * lane + t) * w;
-  }
 #pragma unroll
   for (int t = 0; t < DPL; ++t) st_f<COH>(out + (size_t)h * HD + DPL * lane + t, acc[t] / L);
 }
@@ -118,9 +115,9 @@ IEK_DEV void merge_if_last(const float* __restrict__ part, float* __restrict__ o
   const bool wide = WIDE && nlive - s0 > B1 && (HD >= 256 || nlive - s0 <= 2 * B1);
   for (int g = gb + wave; g < gb + gn; g += 4) {
     if (WIDE && wide)
-      merge_head<HD, COH, 2 * B1>(part, out, kvh * G + g, nsplit, s0, nlive, wsl + 256 * wave);
+      merge_head<HD, COH, 2 * B1>(part, out, kvh * G + g, nsplit, s0, nlive, wsl + MERGE_SLOTS * wave);
     else
-      merge_head<HD, COH, B1>(part, out, kvh * G + g, nsplit, s0, nlive, wsl + 256 * wave);
+      merge_head<HD, COH, B1>(part, out, kvh * G + g, nsplit, s0, nlive, wsl + MERGE_SLOTS * wave);
   }
 }
 
@@ -133,7 +130,7 @@ struct AttnSmem {
   static constexpr int KROW = HD + 16 / ES;  // padded K row: 16 bytes
   static constexpr size_t KS1 = (size_t)SPLIT * KROW * ES, VS1 = (size_t)SPLIT * HD * ES;
   static constexpr size_t KS = SETS * KS1, VS = SETS * VS1, QS = 8 * (size_t)HD * 4, PS = 4 * SETS * SPLIT * 4,
-                          WS = 4 * 256 * 4;
+                          WS = 4 * MERGE_SLOTS * 4;
   static constexpr size_t BYTES = KS + VS + QS + PS + WS + 16;
   T* ks;
   T* vs;
@@ -459,7 +456,7 @@ struct AttnWide {
   static constexpr int UNIT = 4 * KI;  // keys of one step of the workgroup's four waves
   float o[4][4][HD];
   float m[4][4], l[4][4];
-  float wsl[4 * 256];
+  float wsl[4 * MERGE_SLOTS];
   int last;
 };
 

@@ -186,6 +186,26 @@ def test_dev_attention_decode_wide_heads(gpu, kv_f32, n_heads, n_kv, hd, total, 
     test_dev_attention_decode_matches_oracle(gpu, kv_f32, n_heads, n_kv, hd, total, window)
 
 
+@pytest.mark.parametrize("n_heads,hd,total,window", [(2, 256, 131073, 0), (3, 256, 200000, 140001), (1, 512, 200000, 0),
+                                                     (8, 512, 140000, 0)])
+def test_dev_attention_decode_wide_heads_long_context(gpu, n_heads, hd, total, window):
+    """More keys than 256 chunks of sqrt(2 * keys) hold, against float64: every live chunk counts in
+    the maximum and the sum of the merge, and the largest score is in the last of them. Bound as above
+    (f32 sums of 2e5 weights by halves: under 1e-6)."""
+    g = torch.Generator(device="cuda").manual_seed(total + hd)
+    rand = lambda *s: torch.randn(*s, generator=g, device="cuda")  # noqa: E731
+    q, k, v = rand(n_heads, hd), rand(total, hd).half(), rand(total, hd).half()
+    scale = 1.0 / math.sqrt(hd)
+    k[-3] = (q[0] * (10.0 / float(q[0].square().sum() * scale))).half()  # score 10: e^10 of ~3e5 in all
+    lo = max(0, total - window) if window else 0
+    p = torch.softmax((q.double() @ k[lo:].double().T.contiguous()) * scale, 1)
+    want = (p @ v[lo:].double()).cpu().numpy()
+    out = torch.empty(n_heads, hd, device="cuda")
+    E.attention_decode(q.data_ptr(), k.data_ptr(), v.data_ptr(), E.F16, n_heads, 1, hd, total, total, window, scale,
+                       out.data_ptr(), torch.cuda.current_stream().cuda_stream)
+    assert rel_l2(out.cpu().numpy(), want) < 2e-6
+
+
 @pytest.mark.parametrize("totals", [(40, 4000, 41), (3000, 65, 3001, 66, 9000, 67)])
 def test_waiting_entries_share_scratch_between_threads(gpu, totals):
     """The waiting entries keep their scratch for the next call: sizes that grow and shrink, decode

@@ -473,11 +473,13 @@ __global__ __launch_bounds__(64 * WGM * WGN, OCC) void gemm_kq_kernel(GemmQArgs 
   const int lr = lane & 15, lg = lane >> 4;
 
   // Operand streams as buffer loads: one descriptor per array, 32-bit per-lane offsets, the
-  // stage's advance in the scalar offset.
+  // stage's advance in the scalar offset. The activation's start at the tile's rows, so that planes
+  // past 4 GB stay within them.
   const __amdgpu_buffer_rsrc_t rw = buf_rsrc(w, (uint32_t)(g.row_bytes * (size_t)N));
   const __amdgpu_buffer_rsrc_t rw2 = GLU ? buf_rsrc(g.w[1], (uint32_t)(g.row_bytes * (size_t)N)) : rw;
-  const __amdgpu_buffer_rsrc_t rxh = buf_rsrc(g.xh, (uint32_t)(plane_halves(M, K) * 2));
-  const __amdgpu_buffer_rsrc_t rxl = buf_rsrc(g.xl, (uint32_t)(plane_halves(M, K) * 2));
+  const uint32_t xbytes = (uint32_t)(plane_halves(min(BM, M - m0), K) * 2);
+  const __amdgpu_buffer_rsrc_t rxh = buf_rsrc(g.xh + (size_t)m0 * K, xbytes);
+  const __amdgpu_buffer_rsrc_t rxl = buf_rsrc(g.xl + (size_t)m0 * K, xbytes);
   const __amdgpu_buffer_rsrc_t rxs = buf_rsrc(g.xs, T::MINS ? (uint32_t)((size_t)M * kb * 4) : 0u);
   uint32_t vb[4];  // weight row of the lane's column in each 16-column tile
 #pragma unroll
@@ -492,7 +494,7 @@ __global__ __launch_bounds__(64 * WGM * WGN, OCC) void gemm_kq_kernel(GemmQArgs 
     const int i = tid + NT * u;
     as_row[u] = 16 * (i >> 7) + ((i & 63) >> 2);
     as_c[u] = 4 * ((i >> 6) & 1) + (i & 3);
-    const int rt = min((m0 >> 4) + (i >> 7), (M - 1) >> 4);
+    const int rt = min(i >> 7, (M - 1 - m0) >> 4);
     va[u] = (((uint32_t)rt * kb + ((i >> 6) & 1)) * 64 + (i & 63)) * 16u;
   }
   uint32_t vx[TM];  // per-32 sums: k group 0 reads the hi plane, 1 the lo plane

@@ -169,6 +169,22 @@ def test_gemm_few_rows_full_f32_range(gpu, dt, k, n, m):
     _check_matmul(dt, k, n, m, seed=6, a=_wide_range_rows(m, k, 60 + dt))
 
 
+@pytest.mark.parametrize("dt,k,m", [(E.Q4K, 4096, 524287), (E.Q6K, 14336, 149900)])
+def test_gemm_planes_past_4gb(gpu, dt, k, m):
+    """A prompt GEMM whose fp16 planes pass 4 GB, with the padding of the last row tile alone (the first
+    case) or without it: every row against float64, within the relative bar of the other GEMMs."""
+    n = 64
+    w = _weights(dt, k, n, 9)
+    a = torch.randn(m, k, generator=torch.Generator(device="cuda").manual_seed(k), device="cuda")
+    d_w, out = dev(w), torch.empty(m, n, device="cuda")
+    E.matmul(a.data_ptr(), m, k, dt, d_w.data_ptr(), w.nbytes, n, out.data_ptr(), _stream())
+    wt = torch.from_numpy(O.dequantize(ORC[dt], w, k * n // E.BLOCK[dt][0]).reshape(n, k)).to("cuda").double().T.contiguous()
+    for r in range(0, m, 32768):
+        want = a[r:r + 32768].double() @ wt
+        err = (out[r:r + 32768].double() - want).norm(dim=1) / want.norm(dim=1)
+        assert float(err.max()) < 1e-5, r
+
+
 def _wide_range_rows(m, k, seed):
     """Activations over the f32 range the reference takes (src/ops/matmul.rs:176-204 multiplies any
     finite f32): row r is N(0, 1) scaled by 10^(-3 + 9 r / (m - 1)), up to 1e6; every 8th row also

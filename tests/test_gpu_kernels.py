@@ -209,7 +209,9 @@ def test_gemm_parity_full_f32_range(gpu, dt, k, n, m):
     # tile GEMMs whose row factors come with the added halves (K split), in a pass of their own (M * N
     # not a multiple of 4, or one superblock) and in the epilogue (Q8_0), at ragged columns and rows
     (E.Q4K, 512, 300, 260), (E.Q4K, 512, 301, 261), (E.Q4K, 256, 300, 131), (E.Q6K, 1536, 259, 260), (E.Q6K, 768, 65, 257),
-    (E.Q8_0, 96, 301, 129), (E.Q8_0, 2048, 130, 200)])
+    (E.Q8_0, 96, 301, 129), (E.Q8_0, 2048, 130, 200),
+    # rows of one, one and a bit, all and more than all of the chunks that stay in registers
+    (E.Q8_0, 2080, 33, 10), (E.Q8_0, 16384, 40, 9), (E.Q8_0, 16416, 40, 9)])
 def test_gemm_row_factors(gpu, dt, k, n, m):
     _check_matmul(dt, k, n, m, seed=7, a=_wide_range_rows(m, k, 70 + dt))
 

@@ -143,16 +143,15 @@ struct Deq<DT_F32> {
 };
 
 // ---- stage helpers ----------------------------------------------------------------------------
-// activation pair rows m0 .. m0+BM-1 (clamped to M-1), K columns k0 .. k0+31: AU uint4 per plane
+// activation pair rows m0 .. m0+BM-1 (clamped to M-1), K columns k0 .. k0+31: AU uint4 per plane;
+// off: the thread's halves at k0 = 0 (32 columns on are one 16 x 32 tile on)
 template <int AU>
-IEK_DEV void fetch_a(const __half* xh, const __half* xl, int m0, int M, int K, int k0, int tid, u4_t (&arh)[AU],
+IEK_DEV void fetch_a(const __half* xh, const __half* xl, const size_t (&off)[AU], int k0, u4_t (&arh)[AU],
                      u4_t (&arl)[AU]) {
 #pragma unroll
   for (int u = 0; u < AU; ++u) {
-    const int idx = tid + 256 * u, row = idx >> 2, c8 = idx & 3;
-    const size_t off = 8 * plane_chunk(min(m0 + row, M - 1), k0 / 8 + c8, K / 32);
-    arh[u] = *reinterpret_cast<const u4_t*>(xh + off);
-    arl[u] = *reinterpret_cast<const u4_t*>(xl + off);
+    arh[u] = *reinterpret_cast<const u4_t*>(xh + off[u] + (size_t)16 * k0);
+    arl[u] = *reinterpret_cast<const u4_t*>(xl + off[u] + (size_t)16 * k0);
   }
 }
 
@@ -209,7 +208,14 @@ __global__ __launch_bounds__(256) void gemm_mfma_kernel(const uint8_t* __restric
   // per-thread staging assignments
   const int b_row = tid >> 2, b_run = tid & 3;  // weight row within the tile, 8-element run
   const size_t b_f = (size_t)min(n0 + b_row, N - 1) * K + 8 * b_run;
-  u4_t arh[AU], arl[AU];
+  size_t a_off[AU];
+#pragma unroll
+  for (int u = 0; u < AU; ++u)
+    a_off[u] = 8 * plane_chunk(min(m0 + ((tid + 256 * u) >> 2), M - 1), tid & 3, K / 32);
+  struct ASlot {
+    u4_t h[AU], l[AU];
+  };
+  ASlot a0, a1;
   Deq<DT> braw;
   f4_t acc[MT][NT];
 #pragma unroll
@@ -217,18 +223,22 @@ __global__ __launch_bounds__(256) void gemm_mfma_kernel(const uint8_t* __restric
 #pragma unroll
     for (int j = 0; j < NT; ++j) acc[i][j] = f4_t{0.f, 0.f, 0.f, 0.f};
 
-  fetch_a<AU>(xh, xl, m0, M, K, 0, tid, arh, arl);
+  fetch_a<AU>(xh, xl, a_off, 0, a0.h, a0.l);
   braw.raw_load(w, b_f);
-  stage_a<BM, AU>(as_h, as_l, tid, arh, arl);
+  fetch_a<AU>(xh, xl, a_off, min(1, nk - 1) * MBK, a1.h, a1.l);
+  stage_a<BM, AU>(as_h, as_l, tid, a0.h, a0.l);
   stage_b<DT>(bs_h, bs_l, b_row, b_run, braw, b_f);
   __syncthreads();
   const int fr = lane & 15, fk = 8 * (lane >> 4);
-  for (int kt = 0; kt < nk; ++kt) {
-    {
-      const int k1 = min(kt + 1, nk - 1) * MBK;
-      fetch_a<AU>(xh, xl, m0, M, K, k1, tid, arh, arl);
-      braw.raw_load(w, b_f + k1);
-    }
+  // Stage kt: the next stage's weights and the activation of the one after it (into `far`) go out;
+  // `near` holds the next stage's. In the planes' tile order a stage of activation is whole cache lines
+  // that no earlier stage has touched, and one stage ahead does not cover their latency: 24 rows of
+  // Q6_K 512 x 1408 took 55.5 us (51 with row-major planes, whose lines served two stages), now 47.7;
+  // 400 rows of Q4_K 53.4 (52.3), now 46.0; F32 512 x 512 x 4096 126 (131), now 107.
+  auto stage = [&](int kt, ASlot& far, const ASlot& near) {
+    braw.raw_load(w, b_f + min(kt + 1, nk - 1) * MBK);
+    __builtin_amdgcn_sched_barrier(0);
+    fetch_a<AU>(xh, xl, a_off, min(kt + 2, nk - 1) * MBK, far.h, far.l);
     u4_t ah[MT], al[MT], bh[NT], bl[NT];
 #pragma unroll
     for (int i = 0; i < MT; ++i) {
@@ -252,10 +262,14 @@ __global__ __launch_bounds__(256) void gemm_mfma_kernel(const uint8_t* __restric
       }
     __syncthreads();
     if (kt + 1 < nk) {
-      stage_a<BM, AU>(as_h, as_l, tid, arh, arl);
+      stage_a<BM, AU>(as_h, as_l, tid, near.h, near.l);
       stage_b<DT>(bs_h, bs_l, b_row, b_run, braw, b_f + (size_t)(kt + 1) * MBK);
     }
     __syncthreads();
+  };
+  for (int kt = 0; kt < nk; kt += 2) {
+    stage(kt, a0, a1);
+    if (kt + 1 < nk) stage(kt + 1, a1, a0);
   }
 
   // D layout of the 16x16 MFMA: lane holds column lane % 16, rows 4 * (lane / 16) + r

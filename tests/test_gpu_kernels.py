@@ -143,6 +143,15 @@ def test_gemm_parity_mistral_shapes_m512(gpu, dt, k, n):
 
 
 @pytest.mark.parametrize("dt,k,n,m", [
+    # tiles of 128 and 256 rows that keep two stages of K in flight: one, two, three and an odd number
+    # of stages, ragged rows and columns
+    (E.F32, 32, 40, 5), (E.F32, 64, 64, 130), (E.F32, 96, 70, 300), (E.F32, 1056, 65, 129), (E.Q4K, 288, 64, 257),
+    (E.Q6K, 352, 96, 31), (E.Q6K, 352, 2048, 2051)])
+def test_gemm_dequantising_tiles(gpu, dt, k, n, m):
+    _check_matmul(dt, k, n, m, seed=4)
+
+
+@pytest.mark.parametrize("dt,k,n,m", [
     # few-row kernel: the packed-plane tile (up to 8 rows), one, two and four row tiles and their edges
     *[(E.Q4K, 1024, 100, m) for m in (2, 8, 9, 16, 17, 32, 33, 64)],
     # one superblock (a K wave without units), odd counts, K split over workgroups, ragged columns

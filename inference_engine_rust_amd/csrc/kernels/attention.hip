@@ -479,8 +479,8 @@ __global__ __launch_bounds__(256) void attn_prep_kernel(float* __restrict__ q, c
 // CU (NW = 4) or gives eight waves one staged block (NW = 8). Every product takes three MFMAs (hi*hi + hi*lo + lo*hi of the fp16 pairs, exact in f32);
 // the softmax is the online form per query. The longest (latest) query tiles are dispatched first.
 // KG = 2: two sets of NW waves take the tile's key blocks in turn, each with its own staged block,
-// and the second set's (max, sum, O) are folded in through LDS at the end (head_dim 256, whose
-// grids leave most CUs idle: 800 rows of 8 query heads are 100 workgroups). `ovf` (when q was not
+// and the second set's (max, sum, O) are folded in through LDS at the end (head_dim 256 where the
+// grid leaves CUs idle: 800 rows of 8 query heads are 100 workgroups). `ovf` (when q was not
 // checked before): set when a q value is beyond the fp16 pair's range.
 template <int HD, int TMQ, int NW, int KB, int KG = 1>
 __global__ __launch_bounds__(64 * NW * KG, 8 / (NW * KG) > 0 ? 8 / (NW * KG) : 1) void attn_prefill_gqa_kernel(const float* __restrict__ q,
@@ -889,9 +889,13 @@ void launch_attn_prefill(const float* q, const float* k, const float* v, float* 
     // rows: 146 against 176; four waves of two tiles 171)
     const bool wide = wgs(tile(2, 8)) >= 2 * (size_t)num_cus();
     if (head_dim == 256) {
-      // 32-key blocks (the K and V^T planes of a block take 75 KB); one set of four waves took 60 us
-      // for 800 rows of 8 heads and 66 us for 2045, two sets 50 and 55
-      IEK_GQA(256, 1, 4, 32, 2);
+      // 32-key blocks (the K and V^T planes of a block take 75 KB). Two sets of four waves while the
+      // grid holds at most two workgroups per CU, which is what fits of one set: whole calls at 8
+      // heads of one KV head, one set / two, us: 2045 rows (256 workgroups) 215 / 172, 4096 (512) 411 /
+      // 331, window 512 121 / 118, 5000 (626) 500 / 514, 6500 (814) 665 / 807, 8192 (1024) 980 / 1139; 32
+      // heads of 8, 2045 rows (1024) 288 / 341.
+      if (wgs(tile(1, 4)) <= 2 * (size_t)num_cus()) IEK_GQA(256, 1, 4, 32, 2);
+      else IEK_GQA(256, 1, 4, 32, 1);
     } else if (head_dim == 128) {
       if (wide) IEK_GQA(128, 2, 8, 64, 1);
       else IEK_GQA(128, 1, 4, 64, 1);

@@ -303,10 +303,12 @@ def test_dev_attention_prefill_matches_oracle(gpu, n_heads, n_kv, hd, seq, windo
 
 
 @pytest.mark.parametrize("n_heads,n_kv,seq,window", [(8, 1, 1, 0), (8, 1, 31, 0), (8, 1, 33, 0), (4, 2, 65, 16),
-                                                     (3, 1, 96, 33), (8, 8, 129, 0), (8, 1, 577, 512)])
+                                                     (3, 1, 96, 33), (8, 8, 129, 0), (8, 1, 577, 512),
+                                                     (32, 8, 1030, 0), (16, 2, 2065, 50)])
 def test_dev_attention_prefill_key_sets(gpu, n_heads, n_kv, seq, window):
     """head_dim 256: the two wave sets that take the key blocks in turn, at block edges (32 keys),
-    with an odd block count, a window that skips blocks and query groups that leave waves idle."""
+    with an odd block count, a window that skips blocks and query groups that leave waves idle; and the
+    single set of a grid past two workgroups per CU (the last two)."""
     test_dev_attention_prefill_matches_oracle(gpu, n_heads, n_kv, 256, seq, window)
 
 

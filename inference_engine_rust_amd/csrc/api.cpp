@@ -48,121 +48,137 @@ static hipStream_t as_stream(void* s) { return static_cast<hipStream_t>(s); }
 
 static void after_launch() { IEK_HIP(hipGetLastError()); }
 
-// Scratch of the device entries that wait for their stream before they return: a device block and
-// one word of pinned host memory that kernels may store to. A call has its block to itself, and a
-// block is put by for the next call only once the call has waited for its stream (`waited`), so
-// calls of several threads and streams never share one; otherwise it is freed, which waits for the
+// Scratch of the device entries that wait for their stream before they return: a device block and, if
+// asked for, one word of pinned host memory that kernels may store to. A call has them to itself, and
+// they are put by for the next call only once the call has waited for its stream (`waited`), so calls
+// of several threads and streams never share them; otherwise they are freed, which waits for the
 // device. With hipMalloc and hipFree in every call a decode attention of 531 keys took 25.4 us (now
-// 22.8), a prefill attention of 2045 x 32 heads of 128 203 (160), of 800 x 8 heads of 256 80 (68). Kept blocks are bounded per device in bytes and number (the oldest go),
-// and all are given back when a model is freed or an allocation here fails.
-// The block starts with SCRATCH_COUNTERS bytes of arrival counters: zero, and left zero by kernels.
+// 22.8), a prefill attention of 2045 x 32 heads of 128 203 (160), of 800 x 8 heads of 256 80 (68).
+// What is kept is bounded per device in bytes and number (the oldest blocks go; one larger than the
+// bound is never kept and displaces none), and all is given back when a model is freed or an
+// allocation here fails.
+// The block starts with COUNTERS bytes of arrival counters: zero, and left zero by kernels.
 class Scratch {
  public:
   static constexpr size_t COUNTERS = 2 * 4096 * 4;  // two per KV head, at most 4096 heads
-  Scratch(size_t bytes, hipStream_t st) {
+  Scratch(size_t bytes, hipStream_t st, bool word = false) {
     IEK_HIP(hipGetDevice(&b_.device));
     const size_t need = COUNTERS + bytes;
-    {
-      std::lock_guard<std::mutex> lk(mu());
-      auto& k = kept();
-      auto best = k.end();
-      for (auto i = k.begin(); i != k.end(); ++i)
-        if (i->device == b_.device && i->cap >= need && (best == k.end() || i->cap < best->cap)) best = i;
-      if (best != k.end()) {
-        b_ = *best;
-        k.erase(best);
-        return;
-      }
-    }
-    // rounded up by up to a quarter, so that a length that grows call by call keeps its block
-    size_t step = 64 << 10;
-    while (step * 8 <= need) step *= 2;
-    b_.cap = (need + step - 1) / step * step;
-    if (hipMalloc(&b_.dev, b_.cap) != hipSuccess) {
-      (void)hipGetLastError();
-      b_.dev = nullptr;
-      give_back();
-      IEK_HIP(hipMalloc(&b_.dev, b_.cap));
-    }
+    const bool fresh = !take(kept().blocks, b_, [&](const Block& x) { return x.cap >= need; });
     try {
-      IEK_HIP(hipHostMalloc(reinterpret_cast<void**>(&b_.host), 64, hipHostMallocDefault));
-      launch_fill_i32(reinterpret_cast<int*>(b_.dev), 0, COUNTERS / 4, st);
-      after_launch();
+      if (fresh) alloc(need, st);
+      if (word && !take(kept().words, w_, [](const Block&) { return true; })) {
+        w_.device = b_.device;
+        IEK_HIP(hipHostMalloc(&w_.p, 64, hipHostMallocDefault));
+      }
     } catch (...) {
-      release(b_);
+      free_all();
       throw;
     }
   }
   Scratch(const Scratch&) = delete;
   Scratch& operator=(const Scratch&) = delete;
   ~Scratch() {
-    if (!waited_) {
-      release(b_);
-      return;
+    if (waited_) {
+      if (b_.cap <= KEEP_BYTES) keep(kept().blocks, b_);
+      if (w_.p) keep(kept().words, w_);
     }
-    std::vector<Block> drop;
-    bool held = false;
-    try {
-      std::lock_guard<std::mutex> lk(mu());
-      auto& k = kept();
-      k.push_back(b_);
-      held = true;
-      size_t bytes = 0, n = 0;
-      for (auto& x : k)
-        if (x.device == b_.device) bytes += x.cap, ++n;
-      drop.reserve(n);
-      for (auto i = k.begin(); i != k.end() && (bytes > KEEP_BYTES || n > KEEP_BLOCKS);) {
-        if (i->device != b_.device) {
-          ++i;
-          continue;
-        }
-        bytes -= i->cap, --n;
-        drop.push_back(*i);
-        i = k.erase(i);
-      }
-    } catch (const std::bad_alloc&) {  // not kept, or kept beyond the bound until the next call
-      if (!held) drop.clear(), release(b_);
-    }
-    for (auto& x : drop) release(x);
+    free_all();
   }
-  // The call's work on the block is done.
+  // The call's work on the scratch is done.
   void waited() { waited_ = true; }
   template <class T>
   T* at(size_t byte_off = 0) const {
-    return reinterpret_cast<T*>(b_.dev + COUNTERS + byte_off);
+    return reinterpret_cast<T*>(static_cast<char*>(b_.p) + COUNTERS + byte_off);
   }
-  int* counters() const { return reinterpret_cast<int*>(b_.dev); }
-  volatile int* host() const { return b_.host; }
+  int* counters() const { return static_cast<int*>(b_.p); }
+  volatile int* host() const { return static_cast<int*>(w_.p); }
   static void give_back() {
-    std::vector<Block> all;
+    std::vector<Block> b, w;
     {
-      std::lock_guard<std::mutex> lk(mu());
-      all.swap(kept());
+      std::lock_guard<std::mutex> lk(kept().mu);
+      b.swap(kept().blocks);
+      w.swap(kept().words);
     }
-    for (auto& x : all) release(x);
+    for (auto& x : b) (void)hipFree(x.p);
+    for (auto& x : w) (void)hipHostFree(x.p);
   }
 
  private:
   struct Block {
-    char* dev = nullptr;
-    int* host = nullptr;
+    void* p = nullptr;
     size_t cap = 0;
     int device = 0;
   };
+  struct Kept {
+    std::mutex mu;
+    std::vector<Block> blocks, words;
+  };
   static constexpr size_t KEEP_BYTES = 64u << 20, KEEP_BLOCKS = 8;
-  static std::mutex& mu() {
-    static std::mutex* m = new std::mutex;  // (never destroyed: calls may outlast static destructors)
-    return *m;
+  static Kept& kept() {
+    static Kept* k = new Kept;  // (never destroyed: calls may outlast static destructors)
+    return *k;
   }
-  static std::vector<Block>& kept() {
-    static auto* v = new std::vector<Block>;
-    return *v;
+  // the smallest kept one of this device that `fits`
+  template <class Fits>
+  bool take(std::vector<Block>& k, Block& out, Fits fits) {
+    std::lock_guard<std::mutex> lk(kept().mu);
+    auto best = k.end();
+    for (auto i = k.begin(); i != k.end(); ++i)
+      if (i->device == b_.device && fits(*i) && (best == k.end() || i->cap < best->cap)) best = i;
+    if (best == k.end()) return false;
+    out = *best;
+    k.erase(best);
+    return true;
   }
-  static void release(const Block& x) {
-    if (x.dev) (void)hipFree(x.dev);
-    if (x.host) (void)hipHostFree(x.host);
+  // puts x by, in place of the oldest ones beyond the bound (left in `drop_`); x is null on return,
+  // unless there was no memory for the list
+  void keep(std::vector<Block>& k, Block& x) {
+    try {
+      std::lock_guard<std::mutex> lk(kept().mu);
+      k.reserve(k.size() + 1);
+      drop_.reserve(k.size() + 1);
+      size_t bytes = x.cap, n = 1;
+      for (auto& y : k)
+        if (y.device == x.device) bytes += y.cap, ++n;
+      for (auto i = k.begin(); i != k.end() && (bytes > KEEP_BYTES || n > KEEP_BLOCKS);) {
+        if (i->device != x.device) {
+          ++i;
+          continue;
+        }
+        bytes -= i->cap, --n;
+        drop_.push_back(*i);
+        i = k.erase(i);
+      }
+      k.push_back(x);
+      x.p = nullptr;
+    } catch (const std::bad_alloc&) {
+    }
+    for (auto& y : drop_) (void)(y.cap ? hipFree(y.p) : hipHostFree(y.p));  // (words have no cap)
+    drop_.clear();
   }
-  Block b_;
+  void alloc(size_t need, hipStream_t st) {
+    // rounded up by up to a quarter, so that a length that grows call by call keeps its block
+    size_t step = 64 << 10;
+    while (step * 8 <= need) step *= 2;
+    b_.cap = (need + step - 1) / step * step;
+    if (b_.cap > KEEP_BYTES) b_.cap = need;
+    if (hipMalloc(&b_.p, b_.cap) != hipSuccess) {
+      (void)hipGetLastError();
+      b_.p = nullptr;
+      give_back();
+      b_.cap = need;
+      IEK_HIP(hipMalloc(&b_.p, b_.cap));
+    }
+    launch_fill_i32(counters(), 0, COUNTERS / 4, st);
+    after_launch();
+  }
+  void free_all() {
+    if (b_.p) (void)hipFree(b_.p);
+    if (w_.p) (void)hipHostFree(w_.p);
+  }
+  Block b_, w_;
+  std::vector<Block> drop_;
   bool waited_ = false;
 };
 
@@ -578,7 +594,7 @@ iek_status iek_dev_attention_prefill(const float* q, const float* k, const float
     // the K / V^T fp16 planes of the shared-K/V kernel (head_dim up to 256); kernels only ever store
     // to the range flag, so it is the scratch's host word (no clearing launch, no copy back)
     const size_t halves = hd <= 256 ? attn_prefill_scratch_halves(M, nkv, hd) : 0;
-    Scratch s(halves * 2, st);
+    Scratch s(halves * 2, st, true);
     *s.host() = 0;
     launch_attn_prefill(q, k, v, out, M, nh, nkv, hd, win, scale, st, halves ? s.at<char>() : nullptr, halves, false,
                         const_cast<int*>(s.host()));

@@ -251,6 +251,30 @@ def test_waiting_entries_share_scratch_between_threads(gpu, totals):
             assert all(torch.equal(a, b) for a, b in zip(r, want))
 
 
+def test_waiting_entries_keep_scratch_past_a_large_call(gpu):
+    """A call whose scratch is larger than what is kept (the K / V planes of 4200 rows x 16 KV heads of
+    128, 69 MB) leaves the kept scratch of the other entries alone and keeps none of its own: the device's
+    free memory is the same after it, and after the next call of the others."""
+    n, hd, seq, total = 16, 128, 4200, 120000
+    q = torch.zeros(seq, n, hd, device="cuda")
+    k = torch.zeros(1, total, hd, device="cuda")
+    out = torch.empty_like(q)
+    stream = torch.cuda.current_stream().cuda_stream
+
+    def decode():  # about 8 MB of partials
+        E.attention_decode(q.data_ptr(), k.data_ptr(), k.data_ptr(), E.F32, 8, 1, hd, total, total, 0, 0.1, out.data_ptr(),
+                           stream)
+        return torch.cuda.mem_get_info()[0]
+
+    def prefill():
+        E.attention_prefill(q.data_ptr(), q.data_ptr(), q.data_ptr(), seq, n, n, hd, 16, 0.1, out.data_ptr(), stream)
+        return torch.cuda.mem_get_info()[0]
+
+    decode(), prefill()
+    free = decode()
+    assert [prefill(), decode(), prefill(), decode()] == [free] * 4
+
+
 def test_attention_decode_errors(gpu):
     q, k, v = _att_inputs(8, 2, 64, 4, 0)
     for args, kind in [((8, 2, 64, 0, 0), "Op"), ((8, 3, 64, 4, 0), "Op"), ((8, 2, 96, 4, 0), "Op"),

@@ -34,18 +34,20 @@ __global__ __launch_bounds__(256 * SETS) void attn_decode_kernel(const float* __
 // such heads. Against slices of 64 keys staged in LDS (two workgroup barriers a slice, every head's
 // wave reading the whole slice back from LDS): 75 keys of one KV head 8.6 -> 6.8 us at 256, 14.8 ->
 // 9.5 at 512; 500 keys of 512 17.4 -> 11.8; 8000 keys 54 -> 28.
-template <int HD, bool EARLY, typename T>
+// The head groups of a KV head are n_kv workgroups apart, so that they share an XCD's L2 when n_kv is a
+// multiple of the 8 XCDs (8 KV heads of 64 query heads, 32000 f32 keys of 256: 176 -> 131 us).
+template <int HD, int NG, bool EARLY, typename T>
 __global__ __launch_bounds__(256) void attn_decode_wide_kernel(const float* __restrict__ q, const T* __restrict__ kc,
                                                                const T* __restrict__ vc, float* __restrict__ part,
                                                                float* __restrict__ out, int* __restrict__ counters,
                                                                int n_heads, int n_kv, int ctx, const int* pos_dev,
                                                                int total, int window, float scale, int nslot, int CK,
-                                                               int HG) {
+                                                               int HG, int first) {
   __shared__ __align__(16) AttnWide<HD> smem;
   asm volatile("" ::"s"(q), "s"(kc), "s"(vc), "s"(part), "s"(out), "s"(counters), "s"(n_heads), "s"(n_kv), "s"(ctx),
-               "s"(pos_dev), "s"(total), "s"(window), "s"(scale), "s"(nslot), "s"(CK), "s"(HG));
-  attn_chunk_wide<HD, EARLY, T>(q, kc, vc, part, out, counters, n_heads, n_kv, ctx, pos_dev, total, window, scale,
-                                nslot, blockIdx.x / HG, blockIdx.y, CK, smem, blockIdx.x % HG, HG);
+               "s"(pos_dev), "s"(total), "s"(window), "s"(scale), "s"(nslot), "s"(CK), "s"(HG), "s"(first));
+  attn_chunk_wide<HD, NG, EARLY, T>(q, kc, vc, part, out, counters, n_heads, n_kv, ctx, pos_dev, total, window, scale,
+                                    nslot, blockIdx.x % n_kv, first + blockIdx.y, CK, smem, blockIdx.x / n_kv, HG);
 }
 
 template <int HD, typename T>
@@ -93,15 +95,29 @@ static void attn_decode_wide(hipStream_t st, const float* q, const T* kc, const 
   // most MERGE_SLOTS live chunks (a window touches one more than its own length holds).
   constexpr int UNIT = AttnWide<HD>::UNIT;
   const int span = window > 0 ? std::min(max_len, window) : max_len, slots = attn_slots(n_heads, HD, max_len);
-  const int keys = std::max({(int)std::sqrt(2.0 * span), (max_len + slots - 1) / slots,
+  // Several KV heads fill the chip with fewer chunks each, and more of them only add launches and
+  // partials: one chunk of all KV heads per CU, two of an fp16 cache once they hold 512 keys. us with
+  // sqrt(2 * keys) / one / two per CU: 16 KV heads of 256, f32, 8000 keys 85 / 48 / 57, fp16 59 / 41 / 43,
+  // 32000 196 / 142 / 120; 32 query heads of 8 KV heads of 512, f32, 32000 273 / 206 / 222. A session's
+  // chunks are sized for its whole cache, of which any part may be live: 32 per KV head remain there.
+  const long long cus = num_cus(), all = (long long)span * n_kv;
+  const long long fill = pos_dev         ? std::min<long long>(all * HG / (2 * cus), (span + 31) / 32)
+                         : sizeof(T) == 4 ? all / cus
+                                          : std::min(all / cus, std::max(512ll, all / (2 * cus)));
+  const int keys = std::max({(int)std::sqrt(2.0 * span), (int)fill, (max_len + slots - 1) / slots,
                              (span + MERGE_SLOTS - 2) / (MERGE_SLOTS - 1)});
   const int CK = (keys + UNIT - 1) / UNIT * UNIT, nchunk = (max_len + CK - 1) / CK;
+  // the first chunk with a live key, where the host knows the length
+  const int first = !pos_dev && window > 0 && total > window ? (total - window) / CK : 0;
   auto go = [&](auto kern) {
-    hipLaunchKernelGGL(kern, dim3(n_kv * HG, nchunk), dim3(256), 0, st, q, kc, vc, part, out, counters, n_heads, n_kv,
-                       ctx, pos_dev, total, window, scale, nchunk, CK, HG);
+    hipLaunchKernelGGL(kern, dim3(n_kv * HG, nchunk - first), dim3(256), 0, st, q, kc, vc, part, out, counters, n_heads,
+                       n_kv, ctx, pos_dev, total, window, scale, nchunk, CK, HG, first);
   };
   // without a window the first step's loads go out before the position is known
-  window <= 0 ? go(attn_decode_wide_kernel<HD, true, T>) : go(attn_decode_wide_kernel<HD, false, T>);
+  if (n_heads == n_kv)
+    window <= 0 ? go(attn_decode_wide_kernel<HD, 1, true, T>) : go(attn_decode_wide_kernel<HD, 1, false, T>);
+  else
+    window <= 0 ? go(attn_decode_wide_kernel<HD, 4, true, T>) : go(attn_decode_wide_kernel<HD, 4, false, T>);
 }
 
 size_t attn_decode_part_floats(int n_heads, int head_dim, int max_len) {

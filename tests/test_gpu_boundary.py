@@ -177,7 +177,10 @@ def test_dev_attention_decode_matches_oracle(gpu, kv_f32, n_heads, n_kv, hd, tot
 @pytest.mark.parametrize("n_heads,n_kv,hd,total,window", [
     (8, 1, 256, 1, 0), (4, 4, 256, 15, 0), (6, 2, 256, 16, 0), (5, 1, 256, 17, 0), (8, 1, 256, 33, 0),
     (14, 2, 256, 700, 50), (8, 1, 256, 65, 17), (8, 1, 256, 513, 512), (8, 1, 512, 7, 0), (2, 2, 512, 8, 0),
-    (8, 1, 512, 9, 0), (3, 1, 512, 33, 0), (8, 1, 512, 200, 41), (7, 1, 512, 1030, 0)])
+    (8, 1, 512, 9, 0), (3, 1, 512, 33, 0), (8, 1, 512, 200, 41), (7, 1, 512, 1030, 0),
+    # several KV heads: chunks by the number of CUs, groups of one head, whole groups of eight on one XCD,
+    # windows whose first live chunk is not the first
+    (16, 16, 256, 3001, 0), (64, 8, 256, 2100, 0), (16, 16, 512, 1500, 700), (64, 8, 512, 1111, 300), (16, 8, 256, 5000, 33)])
 def test_dev_attention_decode_wide_heads(gpu, kv_f32, n_heads, n_kv, hd, total, window):
     """head_dim 256 and 512 around the edges of a wave's step, its quarter of a chunk and the chunks,
     with head groups that fill their four rows and that do not, and live ranges that start inside a

@@ -54,17 +54,28 @@ template <int HD, typename T>
 static void attn_decode_hd(hipStream_t st, const float* q, const T* kc, const T* vc, float* out, float* part,
                            int* counters, int n_heads, int n_kv, int ctx, const int* pos_dev, int total, int window,
                            float scale, int max_len) {
-  // chunks of spc slices (about 32 chunks per KV head); one partial slot per chunk
-  const int spc = attn_slices_per_chunk(max_len, window, 32);
-  const int nchunk = ((max_len + SPLIT - 1) / SPLIT + spc - 1) / spc;
-  // Chunks of several slices (long contexts) run two slice streams per workgroup, and publish their
-  // partials with coherent stores and a relaxed count (no L2 write-back / invalidate around the
-  // arrival, measured faster there; one-slice chunks are faster with plain stores).
-  const bool two = spc >= 2;
   // A group of 8 query heads splits over two workgroups per chunk (four heads each, one per
   // wave) when there are few KV heads to spread over the machine (one KV head: Gemma-4-E2B);
   // each half has its own arrival counter (2 * n_kv counters) and merge.
   const int HG = (n_heads / n_kv == 8 && n_kv < 4) ? 2 : 1;
+  // Chunks of spc slices (about 32 chunks per KV head); one partial slot per chunk. Where the host knows
+  // the length, one-slice chunks only while all KV heads' fit one to a CU, and at most one chunk per CU
+  // (fp16: two). us with chunks of 1 / 2 / 3 / 4 slices at head_dim 128, f32: 8 KV heads, 2000 keys (256
+  // slices in all) 13.8 / 13.1 / 15.6 / 16.1; 16, 1100 (288) 14.1 / 12.1 / 14.3 / 15.0; 16, 2600 (656) 29.9 /
+  // 21.8 / 17.6 / 18.1; 32, 1500 (768) 32.3 / 20.6 / 17.9 / 18.2; fp16: 16, 2000 (512) 18.1 / 12.5 / 13.4 /
+  // 13.8; 32, 2000 (1024) 31.1 / 13.4 / 14.3 / 14.0; 16, 32000 with 512 chunks 50, with 256 59.
+  const int nsl = (max_len + SPLIT - 1) / SPLIT;
+  int spc = attn_slices_per_chunk(max_len, window, 32);
+  if (!pos_dev) {
+    const long long live = window > 0 ? std::min(nsl, (window + SPLIT - 1) / SPLIT + 1) : nsl;
+    const long long all = live * n_kv * HG, cus = num_cus(), fit = cus * (sizeof(T) == 4 ? 1 : 2);
+    spc = std::max({spc, (int)((all + fit - 1) / fit), all > cus ? 2 : 1});
+  }
+  const int nchunk = (nsl + spc - 1) / spc;
+  // Chunks of several slices (long contexts) run two slice streams per workgroup, and publish their
+  // partials with coherent stores and a relaxed count (no L2 write-back / invalidate around the
+  // arrival, measured faster there; one-slice chunks are faster with plain stores).
+  const bool two = spc >= 2;
   auto go = [&](auto kern, int nt) {
     hipLaunchKernelGGL(kern, dim3(n_kv * HG, nchunk), dim3(nt), 0, st, q, kc, vc, part, out, counters, n_heads, n_kv,
                        ctx, pos_dev, total, window, scale, nchunk, spc, HG);

@@ -125,6 +125,7 @@ def test_host_argmax_and_errors(gpu):
 ATT_CASES = [  # n_heads, n_kv, head_dim, total, window
     (32, 8, 128, 1, 0), (32, 8, 128, 37, 0), (32, 8, 128, 700, 0), (32, 8, 128, 3000, 512),
     (8, 1, 256, 300, 0), (8, 1, 512, 130, 64), (8, 2, 64, 65, 0), (4, 4, 128, 64, 0), (16, 2, 256, 2100, 0),
+    (32, 32, 64, 520, 0), (32, 32, 128, 1300, 0), (16, 16, 128, 2100, 1500),  # chunks by the number of CUs
 ]
 
 
@@ -147,7 +148,9 @@ def test_host_attention_decode_matches_oracle(gpu, n_heads, n_kv, hd, total, win
 
 @pytest.mark.parametrize("kv_f32", [False, True])
 @pytest.mark.parametrize("n_heads,n_kv,hd,total,window", [(32, 8, 128, 520, 0), (8, 1, 256, 1500, 1024),
-                                                          (8, 1, 512, 90, 0), (32, 8, 64, 4100, 0)])
+                                                          (8, 1, 512, 90, 0), (32, 8, 64, 4100, 0),
+                                                          (32, 32, 64, 520, 0), (32, 32, 128, 1300, 0),
+                                                          (16, 16, 128, 2100, 1500)])
 def test_dev_attention_decode_matches_oracle(gpu, kv_f32, n_heads, n_kv, hd, total, window):
     """Device entry over the session layout [n_kv][max_seq_len][head_dim]; an fp16 cache is
     compared with the oracle on the fp16-rounded K/V (the rounding is the cache's, not the op's)."""

@@ -79,12 +79,6 @@ struct QDeq<DT_Q6K> {
   }
 };
 
-// The output factors of rows m .. m + 3 (1 without them; rows past M are not written).
-IEK_DEV void row_factors(const float* row_scale, int m, int M, float (&f)[4]) {
-#pragma unroll
-  for (int r = 0; r < 4; ++r) f[r] = row_scale ? row_scale[min(m + r, M - 1)] : 1.f;
-}
-
 template <int DT, int BM, int BN>
 __global__ __launch_bounds__(256) void gemm_q_kernel(GemmQArgs g) {
   constexpr int WM = BM / 4, MT = WM / 16, NT = BN / 16;
@@ -243,9 +237,7 @@ __global__ __launch_bounds__(256) void gemm_q_kernel(GemmQArgs g) {
 
   const float* resid = s == 0 ? g.resid : nullptr;
 #pragma unroll
-  for (int i = 0; i < MT; ++i) {
-    float f[4];
-    row_factors(g.row_scale, m0 + wave * WM + 16 * i + 4 * (lane >> 4), M, f);
+  for (int i = 0; i < MT; ++i)
 #pragma unroll
     for (int j = 0; j < NT; ++j) {
       const int n = n0 + 16 * j + fr;
@@ -253,13 +245,12 @@ __global__ __launch_bounds__(256) void gemm_q_kernel(GemmQArgs g) {
       for (int r = 0; r < 4; ++r) {
         const int m = m0 + wave * WM + 16 * i + 4 * (lane >> 4) + r;
         if (m < M && n < N) {
-          float v = acc[i][j][r] * f[r];
+          float v = acc[i][j][r];
           if (resid) v = resid[(size_t)m * N + n] + v;
           out[(size_t)m * N + n] = v;
         }
       }
     }
-  }
 }
 
 // ---- K-quants: 64 x 64 wave tiles, weights dequantised straight into MFMA operand registers ----
@@ -907,7 +898,10 @@ bool launch_gemm_q(int dt, const GemmQSeg* segs, int nseg, const __half* xh, con
   }
   switch (dt) {
     case DT_Q4K: return gemm_kq<Q4KB>(g, st, defer_add);
-    case DT_Q6K: gemm_q_dt<DT_Q6K>(g, st); return false;
+    case DT_Q6K:
+      if (row_scale) fail(ST_OP, "gemm_q: native Q6_K tiles take no row factors (regroup the rows)");
+      gemm_q_dt<DT_Q6K>(g, st);
+      return false;
     case DT_Q6K_R: return gemm_kq<Q6RB>(g, st, defer_add);
     default: launch_gemm_q80(g, st); return false;
   }

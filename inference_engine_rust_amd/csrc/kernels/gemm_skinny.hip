@@ -509,8 +509,9 @@ __global__ __launch_bounds__(512, 2) void gemm_skinny_kernel(GemmQArgs g) {
 
 // Workgroups that share a column group's K, for t column groups: split until one workgroup per CU
 // and row block, while each still has two units (two per CU measured slower: 14336 x 4096 Q4_K at 4
-// rows 16.1 against 13.9 us). The split does not depend on the rows, so a row's sums keep their
-// order whatever M is.
+// rows 16.1 against 13.9 us). So a split has at most 256 column groups and K parts, and with at most
+// four row blocks (SK_MAX_ROWS) at most SK_MAX_GROUPS counters. It does not depend on the rows: a row's
+// sums keep their order from 9 rows on (up to 8, the packed planes add the lo products at the end).
 int k_split(int t, int K) { return std::max(1, std::min(std::min(num_cus(), 256) / t, (K / 32 + 7) / 8 / 2)); }
 
 template <class F, int MT, bool PK, bool GLU>
@@ -523,8 +524,7 @@ void skinny_launch(GemmQArgs& g, hipStream_t st) {
   if (GLU) t = g.n[0] / 32;
   for (int i = GLU ? 1 : g.nseg; i <= 3; ++i) g.tile_start[i] = t;
   const int mt = (g.M + 16 * MT - 1) / (16 * MT);
-  g.ksplit = g.sk_cnt && g.kpart && t * mt <= SK_MAX_GROUPS ? k_split(t, g.K) : 1;
-  if (g.ksplit > 1 && t * mt * g.ksplit > SK_MAX_GROUPS) fail(ST_OP, "gemm_skinny: too many row blocks");
+  g.ksplit = g.sk_cnt && g.kpart ? k_split(t, g.K) : 1;
   hipLaunchKernelGGL((gemm_skinny_kernel<F, MT, PK, GLU>), dim3(t * g.ksplit, mt), dim3(512), 0, st, g);
 }
 

@@ -277,7 +277,8 @@ iek_status iek_dev_attention_prefill(const float* q, const float* k, const float
                                      void* stream);
 /* No counterpart in the reference. For callers that cannot allocate device memory (code under
  * HIP graph capture, tight serving loops, harnesses that forbid hipMalloc): iek_dev_attention_decode
- * with the same arguments, results and errors, but its partials and arrival counters live in a 16 MiB scratch array the library holds per device until the process ends; it calls no
+ * with the same arguments, results and errors, but its partials and arrival counters live in a 16 MiB
+ * scratch array the library holds per device until the process ends; it calls no
  * allocator and does not wait for the stream. Limit: n_heads * ceil(max_seq_len / 64) *
  * (head_dim + 2) * 4 bytes <= 16 MiB - 4 KiB (e.g. 32 heads of 128 up to 32K keys), IEK_ERR_OP
  * beyond. Every call on a device shares that device's scratch: calls that overlap on one GPU (two

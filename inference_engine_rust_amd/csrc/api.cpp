@@ -456,7 +456,8 @@ static size_t attention_check(size_t n_heads, size_t n_kv, size_t hd, size_t max
 }
 
 // clear: the counters (2 * n_kv ints) are cleared by a small kernel first, so the sequence is safe
-// under stream capture (the kernel leaves them zero again); the length goes by value, and the chunks are sized for it and not for the cache's capacity.
+// under stream capture (the kernel leaves them zero again); the length goes by value, and the chunks
+// are sized for it and not for the cache's capacity.
 static void attention_launch(const float* q, const void* kc, const void* vc, bool kv_f32, size_t n_heads, size_t n_kv,
                              size_t hd, size_t max_len, size_t total, size_t window, float scale, float* out,
                              float* part, int* cnt, bool clear, hipStream_t st) {

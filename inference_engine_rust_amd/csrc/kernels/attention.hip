@@ -503,8 +503,9 @@ __global__ __launch_bounds__(256) void attn_prep_kernel(float* __restrict__ q, c
 // order krow() gives, the lane's keys of block steps 2t and 2t + 1 are exactly the 8 consecutive
 // keys 32t + 8(lane >> 4) .. + 7 that it supplies as the B operand of O^T += V^T P^T. P stays in
 // registers (no LDS round trip, no wave barrier), and 72 KB of LDS lets two workgroups share a
-// CU (NW = 4) or gives eight waves one staged block (NW = 8). Every product takes three MFMAs (hi*hi + hi*lo + lo*hi of the fp16 pairs, exact in f32);
-// the softmax is the online form per query. The longest (latest) query tiles are dispatched first.
+// CU (NW = 4) or gives eight waves one staged block (NW = 8). Every product takes three MFMAs (hi*hi +
+// hi*lo + lo*hi of the fp16 pairs, exact in f32); the softmax is the online form per query. The longest
+// (latest) query tiles are dispatched first.
 // KG = 2: two sets of NW waves take the tile's key blocks in turn, each with its own staged block,
 // and the second set's (max, sum, O) are folded in through LDS at the end (head_dim 256 where the
 // grid leaves CUs idle: 800 rows of 8 query heads are 100 workgroups). `ovf` (when q was not

@@ -1,7 +1,7 @@
 // Decode attention device code over a per-layer KV cache [n_kv][ctx][head_dim] (f32 or fp16
 // elements), used by the decode attention kernels (attention.hip).
-// src/layers/attention.rs:462-655 (decode_attention_layer): split-K flash-decode over 64-key
-// slices, GQA groups sharing one K/V stream, (max, sum, o[]) partials merged per query head.
+// src/layers/attention.rs:462-655 (decode_attention_layer): split-K flash-decode over chunks of keys,
+// GQA groups sharing one K/V stream, (max, sum, o[]) partials merged per query head.
 #pragma once
 #include "common.cuh"
 #include "../iek_internal.h"
@@ -13,14 +13,8 @@ constexpr int SPLIT = 64;
 // are chosen (attention.hip) so that no launch leaves more of them.
 constexpr int MERGE_SLOTS = 256;
 
-// One 256-thread workgroup per (KV head, 64-key slice): the four waves load the slice's K and V
-// rows (fp16) into LDS together in one burst of clamped, unconditional 16-byte loads, then wave w
-// takes query heads w and w+4 of the GQA group. Lane j scores key j against its head (K row from
-// LDS, q broadcast from LDS), the wave forms the slice softmax, and for P.V lane l owns head dims
-// [DPL*l, DPL*l + DPL). Slices publish (max, sum, o[]) partials; the last workgroup of each KV
-// head to finish merges its query heads (counted with an agent-scope acq_rel atomic per KV head).
-// Merge of the live slice partials of query head h by one wave: global (max, sum) over slices,
-// then each lane folds its head dims of every slice with the rescaled weights. One round trip
+// Merge of the live chunk partials of query head h by one wave: global (max, sum) over chunks,
+// then each lane folds its head dims of every chunk with the rescaled weights. One round trip
 // fetches lane s's (max, sum) pair together with the first batch of B o rows; further batches
 // follow only for more than B live slots (at most MERGE_SLOTS). The last workgroup runs this from a cold
 // instruction cache, so the loop over batches is not unrolled, and a whole batch has no branch per row,
@@ -92,16 +86,15 @@ IEK_DEV void merge_head(const float* __restrict__ part, float* __restrict__ out,
   for (int t = 0; t < DPL; ++t) st_f<COH>(out + (size_t)h * HD + DPL * lane + t, acc[t] / L);
 }
 
-// The last workgroup of a KV head to finish merges the group's heads. Release: the workgroup
-// barrier orders every wave's partial stores before thread 0's agent-scope acq_rel add (which
-// writes back this XCD's L2); the last arrival's acquire side invalidates its L2 before the
-// partials are read. The counter is reset for the next launch.
+// The last workgroup to arrive on counters[cidx] merges query heads [gb, gb + gn) of KV head kvh
+// (G query heads per KV head). Release: every wave waits for its partial stores and the workgroup
+// barrier puts them before thread 0's agent-scope acq_rel add (which writes back this XCD's L2); the
+// last arrival's acquire side invalidates its L2 before the partials are read. With COH the stores are
+// coherent themselves and the count is relaxed. The counter is reset for the next launch.
 // s0 .. nlive-1 are the live partial slots of the KV head. WIDE: twice the batch when that fetches
 // the live slots in one round trip (many-slot merges), and at head_dim 256 and up, whose batches are
 // few rows, for all but the smallest.
 template <int HD, bool COH = false, bool WIDE = false>
-// The last workgroup to arrive on counters[cidx] merges query heads [gb, gb + gn) of KV head kvh
-// (G query heads per KV head).
 IEK_DEV void merge_if_last(const float* __restrict__ part, float* __restrict__ out, int* __restrict__ counters,
                            int kvh, int G, int nsplit, int s0, int nlive, int wave, int* last_s, float* wsl,
                            int gb = 0, int gn = -1, int cidx = -1) {
@@ -212,11 +205,12 @@ IEK_DEV void kv_load(const __half* p, float* f) {
   }
 }
 
-// head_dim 64 and 128: one (KV head, head group, chunk) item of the decode attention over an f32 or fp16 cache (T), by
-// one 256-thread workgroup: the chunk is `spc` consecutive 64-key slices. Each slice's K and V
-// rows are loaded in one burst of clamped, unconditional 16-byte loads and staged in LDS; the
-// loads of slice i+1 are in flight while slice i is computed. The GQA group's G query heads split into HG head groups of G / HG (one workgroup each,
-// all streaming the same K / V); wave w takes heads w and w+4 of its group: lane = key for the
+// head_dim 64 and 128: one (KV head, head group, chunk) item of the decode attention over an f32 or
+// fp16 cache (T), by one 256-thread workgroup: the chunk is `spc` consecutive 64-key slices. Each
+// slice's K and V rows are loaded in one burst of clamped, unconditional 16-byte loads and staged in
+// LDS; the loads of slice i+1 are in flight while slice i is computed. The GQA group's G query heads
+// split into HG head groups of G / HG (one workgroup each, all streaming the same K / V); wave w takes
+// heads w and w+4 of its group: lane = key for the
 // scores, lane = head dims [DPL*l, DPL*l + DPL) for P.V, with a running (max, sum, o) across the
 // chunk's slices. The chunk publishes its (max, sum, o[]) partials in slot `cp`; the last chunk
 // of the (KV head, head group) to finish merges the group's heads (counter kvh * HG + hg).
@@ -649,8 +643,8 @@ IEK_DEV void attn_chunk_wide(const float* __restrict__ q, const T* __restrict__ 
     }
   }
   if (nslot == 1) return;
-  merge_if_last<HD, false, true>(part, out, counters, kvh, G, nslot, jmin / CK, (total + CK - 1) / CK, wave, &S.last, S.wsl, gb, GH,
-                    kvh * HG + hg);
+  merge_if_last<HD, false, true>(part, out, counters, kvh, G, nslot, jmin / CK, (total + CK - 1) / CK, wave, &S.last,
+                                 S.wsl, gb, GH, kvh * HG + hg);
 }
 
 // Slices per chunk for a cache of `max_len` keys: one up to `target` slices per KV head, then

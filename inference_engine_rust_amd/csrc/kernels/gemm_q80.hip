@@ -9,10 +9,10 @@
 //
 // Against the tiles it took over from (64 x 64 with both operands staged through LDS as fp16, a wave
 // of 16 x 64 reading six LDS operands for eight MFMAs, one barrier per 32 of K), whole op-level calls,
-// us: 256 x 6144 x 1536 45.8 -> 33.5; 130 x 4096 x 14336 229 -> 93; 256 x 1536 x 6144 110 -> 50;
+// us: 256 x 6144 x 1536 42.0 -> 29.0; 130 x 4096 x 14336 229 -> 93; 256 x 1536 x 6144 110 -> 50;
 // 512 x 14336 x 4096 279 -> 194. With tiles left over the bound is a wave's chain of steps (~0.8 us
 // per 32 of K with one wave per SIMD); prefetching the activation two blocks ahead instead of one
-// changed nothing (33.5 / 34.0, 98 / 99), so it is not the loads' latency.
+// changed nothing (98 / 99 at 130 x 4096 x 14336), so it is not the loads' latency.
 #include <algorithm>
 
 #include "kq_core.cuh"

@@ -552,14 +552,23 @@ void skinny(GemmQArgs& g, bool glu, hipStream_t st) {
 
 // Few rows: every output column of up to 64 rows costs this kernel one pass over the weights, where
 // the 64 x 256 tiles of gemm_q.hip cost the same for 64 rows as for one until they fill the chip.
-// Measured (us, this kernel against that one with its split-K and row-scale passes): Q4_K
-// 4096 x 4096 at 23 rows 13 / 46, 64 rows 22 / 48, 128 rows 30 / 52; 14336 x 4096 at 23 rows 24 / 48,
-// 64 rows 44 / 46, 128 rows 86 / 57. Q6_K 4096 x 14336 at 23 rows 30 / 220, 64 rows 47 / 221, 128
-// rows 83 / 227 (its tiles take three MFMAs per product and K = 14336 on 32 workgroups). Q8_0
-// 6144 x 1536 at 23 rows 13 / 29; 1536 x 6144 at 13 rows 11 / 92. Q8_0 above 32 rows takes two or
-// more passes of 32 here, and gemm_q80.hip's tiles are as fast once they are enough of them (whole
-// op-level calls, this kernel / those): 64 rows 4096 x 14336 65 / 92, 1536 x 6144 34 / 45, 6144 x 1536
-// 31 / 24, 14336 x 4096 62 / 43; 128 rows 512 x 4096 25 / 38, 1536 x 6144 51 / 49, 1536 x 2048
+// Whole op-level calls, us, this kernel / the tiles with their split-K and row-scale passes, N x K:
+//   Q4_K 4096 x 4096    23 rows 26 / 50   64 30 / 52   65 46 / 52   128 50 / 55   129  66 / 54   256  89 / 59
+//        6144 x 4096                      64 38 / 52   65 62 / 52
+//        14336 x 4096   23 rows 33 / 53   33 51 / 53   64 55 / 55   128 99 / 63
+//        6144 x 1536                      64 27 / 31   65 41 / 32
+//        1024 x 4096                                                128 28 / 51   129  36 / 51   256  43 / 54
+//        4096 x 14336                                               128 102 / 149 192 144 / 149  256 187 / 155
+//   Q6_K 4096 x 14336   23 rows 42 / 265  64 60 / 271  128 105 / 273  256 198 / 275
+//        14336 x 4096                     64 57 / 106  65 98 / 107  128 102 / 112  200 191 / 180
+//        6144 x 1536                      64 28 / 49   128 46 / 52  129  62 / 51   256  66 / 56
+// So this kernel takes any width up to 32 rows (Q6_K, whose tiles take three MFMAs per product, up to
+// 64), and further rows while columns times row blocks stay where it costs less. The lines are on the
+// safe side of where the two cross, not on it: narrow Q4_K at 129 to 256 rows, Q4_K of large K and wide
+// Q6_K above 64 rows stay with the tiles although this kernel is faster there.
+// Q8_0 above 32 rows takes two or more passes of 32 here, and gemm_q80.hip's tiles are as fast once they
+// are enough of them (this kernel / those): 64 rows 4096 x 14336 65 / 92, 1536 x 6144 34 / 45, 6144 x
+// 1536 31 / 24, 14336 x 4096 62 / 43; 128 rows 512 x 4096 25 / 38, 1536 x 6144 51 / 49, 1536 x 2048
 // 28 / 26, 6144 x 1536 41 / 34, 4096 x 14336 113 / 93.
 bool gemm_skinny_ok(int dt, int M, int N) {
   const long long c = (long long)N * ((M + 63) / 64);
